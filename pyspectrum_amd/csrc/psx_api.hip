@@ -6,6 +6,7 @@
 #include <numeric>
 
 #include "psx_ctx.h"
+#include "psx_lattice.h"
 #include "psx_plan.h"
 
 namespace psx {
@@ -246,46 +247,34 @@ int get_shell_plan(psx_ctx* ctx, int N, int step, int ncut, int nmax, int kt, in
 // triangle_list, triangle_cover: psx_plan.h
 
 
-int get_contract_plan(psx_ctx* ctx, int prec, int step, int ncut, int nmax,
-                      const ContractPlan** out);
-
-// Split-BF16 contraction: the LDS serves the 16-byte A reads of 8 rows of a
-// pair tile per cycle, conflict-free when their distinct shells differ
-// modulo 8 (float rows 8 words apart modulo 64 banks).  Swap rows between
-// the two 8-row halves of each tile while that lowers the number of shells
-// that share a bank group with another shell of their half (i and j
-// columns).  Row order inside a tile does not change any result.
-static void arrange_half_tiles(std::vector<int>* prow, int nsh, int j0) {
-  auto half_cost = [&](const int* r) {
-    int c = 0;
-    for (int col = 0; col < 2; ++col) {
-      int seen[64], nseen = 0, grp[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      for (int k = 0; k < 8; ++k) {
-        if (r[k] < 0) continue;
-        const int sh = (col == 0 ? r[k] / nsh : r[k] % nsh) - j0;
-        bool dup = false;
-        for (int m = 0; m < nseen; ++m) dup |= seen[m] == sh;
-        if (dup) continue;
-        seen[nseen++] = sh;
-        c += grp[sh & 7]++ > 0 ? 1 : 0;
-      }
-    }
-    return c;
-  };
-  for (size_t t = 0; t + 16 <= prow->size(); t += 16) {
-    int* r = prow->data() + t;
-    int cur = half_cost(r) + half_cost(r + 8);
-    for (bool improved = true; improved;) {
-      improved = false;
-      for (int a = 0; a < 8; ++a)
-        for (int b = 8; b < 16; ++b) {
-          std::swap(r[a], r[b]);
-          const int c2 = half_cost(r) + half_cost(r + 8);
-          if (c2 < cur) { cur = c2; improved = true; }
-          else std::swap(r[a], r[b]);
-        }
-    }
-  }
+// Contraction plan of the triangles ijl on the shells j0..nmax: the host
+// layout (psx_plan.h) for the kernel of `prec` (with the fused kernel's wave
+// layout if `fused`), uploaded.
+static int build_contract_plan(psx_ctx* ctx, int prec, bool fused, const std::vector<int>& ijl,
+                               int j0, int nmax, ContractPlan* cp) {
+  const int ns = nmax - j0 + 1;
+  const int nlt = (int)cdiv(ns, 16);
+  if (nlt > 4)
+    return set_error(PSX_ERR_UNSUPPORTED, "at most 64 shells (Nmax - Ncut//step + 1 <= 64)");
+  LayoutShape ls;
+  ls.f64 = prec == PSX_PREC_F64;
+  ls.simd_balance = fused;
+  ls.maxpt = fused ? xc_maxpt() : contract_maxpt(prec, nlt);
+  ls.wpg = fused ? xc_waves_per_group() : contract_waves_per_group(prec, nlt);
+  ContractLayout cl;
+  PSX_REQUIRE(contract_layout(ijl, j0, nmax, ls, &cl),
+              "contraction plan: a triangle without a chosen pair");
+  cp->j0 = j0; cp->ns = ns; cp->nmax = nmax; cp->nlt = nlt;
+  cp->ntri = (int)(ijl.size() / 3);
+  cp->npairs = cl.npairs; cp->npt = cl.npt; cp->nblk = cl.nblk; cp->nslot = cl.nslot;
+  cp->waves = cl.waves; cp->maxpt = ls.maxpt;
+  PSX_TRY(upload(ctx, cl.wave_pt, &cp->d_wave_pt));
+  PSX_TRY(upload(ctx, cl.wave_mask, &cp->d_wave_mask));
+  PSX_TRY(upload(ctx, cl.wave_slot, &cp->d_wave_slot));
+  PSX_TRY(upload(ctx, cl.pair_s, &cp->d_pair_s));
+  PSX_TRY(upload(ctx, cl.tri_loc, &cp->d_tri_loc));
+  PSX_TRY(upload(ctx, cl.tri_grp, &cp->d_tri_grp));
+  return PSX_OK;
 }
 
 int get_contract_plan(psx_ctx* ctx, int prec, int step, int ncut, int nmax,
@@ -297,177 +286,75 @@ int get_contract_plan(psx_ctx* ctx, int prec, int step, int ncut, int nmax,
   auto it = ctx->contract_plans.find(key);
   if (it != ctx->contract_plans.end()) { *out = it->second.get(); return PSX_OK; }
   auto cp = std::make_unique<ContractPlan>();
-  const int j0 = ncut / step;
-  const int ns = nmax - j0 + 1;
-  cp->j0 = j0; cp->ns = ns; cp->nmax = nmax;
-  cp->nlt = (int)cdiv(ns, 16);
-  if (cp->nlt > 4)
-    return set_error(PSX_ERR_UNSUPPORTED, "at most 64 shells (Nmax - Ncut//step + 1 <= 64)");
   std::vector<int> ijl;
   triangle_list(step, ncut, nmax, &ijl);
-  cp->ntri = (int)(ijl.size() / 3);
-  std::vector<int> tpair, tshell;
-  triangle_cover(ijl, nmax, j0, &tpair, &tshell);
-  for (int t = 0; t < cp->ntri; ++t)
-    PSX_REQUIRE(tpair[t] >= 0, "contraction plan: a triangle without a chosen pair");
-  // pair tiles: pairs grouped by their set of column tiles, whole tiles of one
-  // set first, the remainders sorted by (tiles used, set) and cut into tiles
-  std::map<int, int> pmask;  // pair key -> column tiles it reads
-  for (int t = 0; t < cp->ntri; ++t) pmask[tpair[t]] |= 1 << ((tshell[t] - j0) / 16);
-  std::map<int, std::vector<int>> by_mask;
-  for (const auto& pm : pmask) by_mask[pm.second].push_back(pm.first);
-  std::vector<int> prow;  // pair key of each row, -1 = padding
-  std::vector<std::pair<int, int>> rest;
-  for (const auto& bm : by_mask) {
-    const size_t whole = bm.second.size() / 16 * 16;
-    prow.insert(prow.end(), bm.second.begin(), bm.second.begin() + whole);
-    for (size_t k = whole; k < bm.second.size(); ++k) rest.push_back({bm.first, bm.second[k]});
-  }
-  std::stable_sort(rest.begin(), rest.end(), [](const std::pair<int, int>& a, const std::pair<int, int>& b) {
-    const int pa = __builtin_popcount(a.first), pb = __builtin_popcount(b.first);
-    return pa != pb ? pa < pb : a.first < b.first;
-  });
-  for (const auto& r : rest) prow.push_back(r.second);
-  cp->npairs = (int)prow.size();
-  cp->npt = (int)cdiv(cp->npairs, 16);
-  prow.resize((size_t)cp->npt * 16, -1);
-  const int nsh = nmax + 1;
-  if (prec != PSX_PREC_F64) arrange_half_tiles(&prow, nsh, j0);
-  std::vector<int> pair_s(2 * prow.size(), -1);
-  std::map<int, int> prow_of;
-  for (size_t r = 0; r < prow.size(); ++r) {
-    if (prow[r] < 0) continue;
-    pair_s[2 * r] = prow[r] / nsh - j0;
-    pair_s[2 * r + 1] = prow[r] % nsh - j0;
-    prow_of[prow[r]] = (int)r;
-  }
-  std::vector<int> ptmask(cp->npt, 0);
-  std::vector<int> tpt(cp->ntri), trow(cp->ntri), tlt(cp->ntri), tcol(cp->ntri);
-  for (int t = 0; t < cp->ntri; ++t) {
-    const int p = prow_of.at(tpair[t]);
-    tpt[t] = p / 16; trow[t] = p % 16;
-    tlt[t] = (tshell[t] - j0) / 16; tcol[t] = (tshell[t] - j0) % 16;
-    ptmask[tpt[t]] |= 1 << tlt[t];
-  }
-  cp->nblk = 0;
-  for (int m : ptmask) cp->nblk += __builtin_popcount(m);
-  // assign pair tiles to waves: groups of WPG waves x maxpt slots, greedy by load
-  const int maxpt = fused ? xc_maxpt() : contract_maxpt(prec, cp->nlt);
-  const int WPG = fused ? xc_waves_per_group() : contract_waves_per_group(prec, cp->nlt);
-  const int ngroups = (int)cdiv(cp->npt, WPG * maxpt);
-  const int nw = ngroups * WPG;
-  std::vector<int> order(cp->npt);
-  std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-    return __builtin_popcount(ptmask[a]) > __builtin_popcount(ptmask[b]);
-  });
-  std::vector<int> load(nw, 0), cnt(nw, 0);
-  std::vector<int> wave_pt(nw * maxpt, -1), wave_mask(nw * maxpt, 0);
-  std::vector<int> pt_wave(cp->npt), pt_q(cp->npt);
-  for (int pt : order) {
-    int best = -1;
-    for (int w = 0; w < nw; ++w)
-      if (cnt[w] < maxpt && (best < 0 || load[w] < load[best])) best = w;
-    wave_pt[best * maxpt + cnt[best]] = pt;
-    wave_mask[best * maxpt + cnt[best]] = ptmask[pt];
-    pt_wave[pt] = best; pt_q[pt] = cnt[best];
-    cnt[best]++;
-    // cost of a tile: forming and splitting its products (about three
-    // blocks' worth of MFMA time) plus its output blocks
-    load[best] += 3 + __builtin_popcount(ptmask[pt]);
-  }
-  // Fused layout (one workgroup per CU): the waves of the workgroup are
-  // spread over the CU's four SIMDs (wave w on SIMD w % 4), and a SIMD issues
-  // its waves' VALU and MFMA work one at a time, so what bounds the group is
-  // the busiest SIMD.  Swap tiles (or a tile and an empty slot) between waves
-  // of different SIMDs while that lowers the group's (largest SIMD load, sum
-  // of squared SIMD loads).  Which wave runs a tile changes no result: its
-  // sums are formed in the same order.  (Measured at Ngrid 360, 40 shells:
-  // k_xcontract 6.13 -> 5.95 ms; the staged k_contract, several workgroups
-  // per CU, ran 4-6 % slower with it and keeps the per-wave balance.)
-  if (fused && WPG % 4 == 0) {
-    auto tcost = [&](int pt) { return pt < 0 ? 0 : 3 + __builtin_popcount(ptmask[pt]); };
-    for (int g = 0; g < ngroups; ++g) {
-      const int w0 = g * WPG;
-      auto score = [&](long long* sq) {
-        int sl[4] = {0, 0, 0, 0};
-        for (int w = w0; w < w0 + WPG; ++w) sl[(w - w0) % 4] += load[w];
-        *sq = 0;
-        int mx = 0;
-        for (int s = 0; s < 4; ++s) { mx = std::max(mx, sl[s]); *sq += (long long)sl[s] * sl[s]; }
-        return mx;
-      };
-      long long sq;
-      int mx = score(&sq);
-      for (bool improved = true; improved;) {
-        improved = false;
-        for (int a = w0 * maxpt; a < (w0 + WPG) * maxpt; ++a)
-          for (int b = a + 1; b < (w0 + WPG) * maxpt; ++b) {
-            const int wa = a / maxpt, wb = b / maxpt;
-            if ((wa - w0) % 4 == (wb - w0) % 4 || wave_pt[a] == wave_pt[b]) continue;
-            const int d = tcost(wave_pt[b]) - tcost(wave_pt[a]);
-            load[wa] += d; load[wb] -= d;
-            long long sq2;
-            const int mx2 = score(&sq2);
-            if (mx2 < mx || (mx2 == mx && sq2 < sq)) {
-              std::swap(wave_pt[a], wave_pt[b]);
-              std::swap(wave_mask[a], wave_mask[b]);
-              mx = mx2; sq = sq2; improved = true;
-            } else {
-              load[wa] -= d; load[wb] += d;
-            }
-          }
-      }
-    }
-    // slots in use first within each wave (the kernels count a wave's tiles)
-    for (int w = 0; w < nw; ++w)
-      for (int q = 0; q < maxpt; ++q)
-        for (int r = q + 1; r < maxpt && wave_pt[w * maxpt + q] < 0; ++r)
-          if (wave_pt[w * maxpt + r] >= 0) {
-            std::swap(wave_pt[w * maxpt + q], wave_pt[w * maxpt + r]);
-            std::swap(wave_mask[w * maxpt + q], wave_mask[w * maxpt + r]);
-          }
-    for (int w = 0; w < nw; ++w)
-      for (int q = 0; q < maxpt; ++q) {
-        const int pt = wave_pt[w * maxpt + q];
-        if (pt >= 0) { pt_wave[pt] = w; pt_q[pt] = q; }
-      }
-  }
-  // output slots per group: the blocks that hold a triangle
-  std::vector<int> wave_slot(nw * maxpt * 4, -1);
-  std::vector<int> gslots(ngroups, 0);
-  for (int w = 0; w < nw; ++w)
-    for (int q = 0; q < maxpt; ++q) {
-      const int pt = wave_pt[w * maxpt + q];
-      for (int t = 0; t < 4; ++t)
-        if (pt >= 0 && ((ptmask[pt] >> t) & 1)) wave_slot[(w * maxpt + q) * 4 + t] = gslots[w / WPG]++;
-    }
-  cp->nslot = *std::max_element(gslots.begin(), gslots.end());
-  std::vector<int> tri_loc(cp->ntri), tri_grp(cp->ntri);
-  for (int t = 0; t < cp->ntri; ++t) {
-    const int w = pt_wave[tpt[t]], q = pt_q[tpt[t]];
-    const int slot = wave_slot[(w * maxpt + q) * 4 + tlt[t]];
-    const int row = trow[t], col = tcol[t];
-    // 16x16 MFMA output layout (measured on gfx950): f32 outputs (f32 and bf16
-    // inputs) hold row r in lane col + 16*(r/4), register r%4; the f64 MFMA
-    // holds it in lane col + 16*(r%4), register r/4.
-    const bool f64 = prec == PSX_PREC_F64;
-    const int lane = col + 16 * (f64 ? row % 4 : row / 4);
-    const int reg = f64 ? row / 4 : row % 4;
-    tri_loc[t] = slot * 256 + lane * 4 + reg;
-    tri_grp[t] = w / WPG;
-  }
-  cp->waves = nw;
-  cp->maxpt = maxpt;
-  PSX_TRY(upload(ctx, wave_pt, &cp->d_wave_pt));
-  PSX_TRY(upload(ctx, wave_mask, &cp->d_wave_mask));
-  PSX_TRY(upload(ctx, wave_slot, &cp->d_wave_slot));
-  PSX_TRY(upload(ctx, pair_s, &cp->d_pair_s));
-  PSX_TRY(upload(ctx, tri_loc, &cp->d_tri_loc));
-  PSX_TRY(upload(ctx, tri_grp, &cp->d_tri_grp));
-  PSX_TRY(upload(ctx, ijl, &cp->d_tri_ijl));
+  PSX_TRY(build_contract_plan(ctx, prec, fused, ijl, ncut / step, nmax, cp.get()));
   *out = cp.get();
   ctx->contract_plans[key] = std::move(cp);
+  return PSX_OK;
+}
+
+// ---------------------------------------------------------- FP64 layers ----
+int get_lattice_plan(psx_ctx* ctx, int N, int step, int ncut, int nmax, const LatticePlan** out) {
+  auto key = std::make_tuple(N, step, ncut, nmax);
+  auto it = ctx->lattice_plans.find(key);
+  if (it != ctx->lattice_plans.end()) { *out = it->second.get(); return PSX_OK; }
+  std::vector<int> ijl, sizes;
+  triangle_list(step, ncut, nmax, &ijl);
+#define PSX_ADD_N(n) sizes.push_back(n);
+  PSX_LAT_SIZES(PSX_ADD_N)
+#undef PSX_ADD_N
+  std::sort(sizes.begin(), sizes.end());
+  bool fast = false;
+#define PSX_IF_N(n) fast = fast || N == n;
+  PSX_FFT_SIZES(PSX_IF_N)
+#undef PSX_IF_N
+  auto lp = std::make_unique<LatticePlan>();
+  for (const LayerChoice& c :
+       choose_layers(ijl, N, [&](int j) { return shell_mmax(j, step); }, sizes, fast)) {
+    LatticeLayer l;
+    l.M = c.M;
+    l.add = c.add;
+    l.ntri = (int)c.tri.size();
+    l.j0 = nmax;
+    for (int t : c.tri) {
+      l.ijl.insert(l.ijl.end(), ijl.begin() + 3 * t, ijl.begin() + 3 * t + 3);
+      l.j0 = std::min(l.j0, ijl[3 * t + 2]);
+      l.nmax = std::max(l.nmax, ijl[3 * t]);
+    }
+    if (c.shifted) {
+      std::vector<c64> ph(c.M / 2 + 1);
+      for (int k = 0; k <= c.M / 2; ++k) {
+        const long double a = -3.141592653589793238462643383279502884L * (long double)k / c.M;
+        ph[k] = mk((double)cosl(a), (double)sinl(a));
+      }
+      c64* d;
+      PSX_TRY(upload(ctx, ph, &d));
+      l.phase = d;
+    }
+    PSX_TRY(upload(ctx, c.tri, &l.d_map));
+    PSX_TRY(upload(ctx, c.weight, &l.d_weight));
+    if (l.ntri > DIRECT_TRI || l.nmax - l.j0 + 1 > DIRECT_SHELLS) {
+      l.cp = std::make_unique<ContractPlan>();
+      PSX_TRY(build_contract_plan(ctx, PSX_PREC_F64, false, l.ijl, l.j0, l.nmax, l.cp.get()));
+    }
+    lp->layers.push_back(std::move(l));
+  }
+  *out = lp.get();
+  ctx->lattice_plans[key] = std::move(lp);
+  return PSX_OK;
+}
+
+// The FP64 triangle sums layer by layer (the shell buffers are reused).
+static int lattice_sums(psx_ctx* ctx, const LatticePlan* lp, const void* half, int N, int step,
+                        double* braw) {
+  for (const LatticeLayer& l : lp->layers) {
+    const size_t n = (size_t)(l.nmax - l.j0 + 1) * l.M * l.M * l.M;
+    void* D;
+    PSX_TRY(ctx_buffer(ctx, "shells", n * sizeof(double), &D));
+    PSX_TRY(launch_lattice_fields(ctx, half, N, step, l, D));
+    PSX_TRY(launch_lattice_sums(ctx, D, l, braw));
+  }
   return PSX_OK;
 }
 
@@ -568,6 +455,11 @@ static int bk_raw_main(psx_ctx* ctx, const void* half, int N, int step, int ncut
     // fields never go through HBM
     PSX_TRY(launch_xcontract(ctx, half, N, step, ncut, nmax, braw));
   } else {
+    if (prec == PSX_PREC_F64) {
+      const LatticePlan* lp;
+      PSX_TRY(get_lattice_plan(ctx, N, step, ncut, nmax, &lp));
+      if (!lp->layers.empty()) return lattice_sums(ctx, lp, half, N, step, braw);
+    }
     void* D;
     PSX_TRY(ctx_buffer(ctx, "shells", (size_t)ns * G * rbytes(fp), &D));
     PSX_TRY(launch_shell_fields(ctx, half, N, step, ncut, nmax, fp, D));
@@ -988,7 +880,9 @@ int psx_bk_workspace_bytes(psx_ctx* ctx, int ngrid, int step, int ncut, int nmax
   PSX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
   const int64_t ngroups =
       cp->waves / (fused ? xc_waves_per_group() : contract_waves_per_group(prec, cp->nlt));
-  b += (8 * (int64_t)cus + ngroups) * cp->nslot * 256 * 8;                // partials, reduction
+  // partials and reduction; the FP64 layers' smaller grids stay within the
+  // fields above, their plans (a block or two more) within the factor 8
+  b += (8 * (int64_t)cus + ngroups) * cp->nslot * 256 * 8 + (256 << 10);
   b += (int64_t)(cp->ntri + 1) * 8 + 513 * 3 * (int64_t)nmax * 8;          // braw, p0k bins
   *bytes = b;
   return PSX_OK;
@@ -1061,14 +955,9 @@ int psx_bk_periodic_batch(psx_ctx* ctx, int nbox, const psx_box* boxes, int ngri
   const int rc = [&]() -> int {
     if (xcontract_supported(ctx, N, step, ncut, nmax, prec) == PSX_OK)
       return launch_xcontract(ctx, half, N, step, ncut, nmax, (double*)braw, nbox);
-    const int ns = nmax - ncut / step + 1;
-    void* D;
-    PSX_TRY(ctx_buffer(ctx, "shells", (size_t)ns * G * rbytes(fp), &D));
-    for (int b = 0; b < nbox; ++b) {
-      PSX_TRY(launch_shell_fields(ctx, (const char*)half + (size_t)b * nh * cbytes(fp), N, step,
-                                  ncut, nmax, fp, D));
-      PSX_TRY(launch_contract(ctx, D, N, step, ncut, nmax, prec, (double*)braw + (size_t)b * ntri));
-    }
+    for (int b = 0; b < nbox; ++b)
+      PSX_TRY(bk_raw_main(ctx, (const char*)half + (size_t)b * nh * cbytes(fp), N, step, ncut, nmax,
+                          (double*)braw + (size_t)b * ntri, prec, fp, nmax - ncut / step + 1, G));
     return PSX_OK;
   }();
   PSX_TRY(join_side(ctx));

@@ -40,6 +40,7 @@
 #include <algorithm>
 
 #include "psx_ctx.h"
+#include "psx_lattice.h"
 #include "psx_mfma.h"
 
 namespace psx {
@@ -435,8 +436,20 @@ __global__ void k_contract_gather(const double* __restrict__ red, int nslot, int
   braw[(int64_t)blockIdx.y * ntri + t] = red[(int64_t)tri_grp[t] * nslot * 256 + tri_loc[t]];
 }
 
+// A layer's sums to their places in the full triangle list, weighted; add:
+// to what an earlier layer left there.
+__global__ void k_layer_gather(const double* __restrict__ red, int nslot,
+                               const int* __restrict__ tri_loc, const int* __restrict__ tri_grp,
+                               const int* __restrict__ map, const double* __restrict__ weight,
+                               int ntri, bool add, double* __restrict__ braw) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= ntri) return;
+  const double v = weight[t] * red[(int64_t)tri_grp[t] * nslot * 256 + tri_loc[t]];
+  braw[map[t]] = add ? braw[map[t]] + v : v;
+}
+
 int launch_contract_reduce(psx_ctx* ctx, const ContractPlan* cp, const double* part, int64_t nwg,
-                           int ngroups, double* braw, int nbox) {
+                           int ngroups, double* braw, int nbox, const LatticeLayer* layer) {
   const int nslot = cp->nslot;
   void* red = nullptr;
   PSX_TRY(ctx_buffer(ctx, "contract_red", (size_t)nbox * ngroups * nslot * 256 * sizeof(double),
@@ -444,9 +457,14 @@ int launch_contract_reduce(psx_ctx* ctx, const ContractPlan* cp, const double* p
   hipLaunchKernelGGL(k_contract_reduce<double>, dim3((unsigned)nslot, 4, nbox * ngroups),
                      dim3(64 * RED_SEG), 0, ctx->stream, part, nwg, nslot, (double*)red);
   PSX_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_contract_gather, dim3((unsigned)cdiv(cp->ntri, 128), nbox), dim3(128), 0,
-                     ctx->stream, (const double*)red, nslot, ngroups, cp->d_tri_loc,
-                     cp->d_tri_grp, cp->ntri, braw);
+  if (layer)
+    hipLaunchKernelGGL(k_layer_gather, dim3((unsigned)cdiv(cp->ntri, 128)), dim3(128), 0,
+                       ctx->stream, (const double*)red, nslot, cp->d_tri_loc, cp->d_tri_grp,
+                       layer->d_map, layer->d_weight, cp->ntri, layer->add, braw);
+  else
+    hipLaunchKernelGGL(k_contract_gather, dim3((unsigned)cdiv(cp->ntri, 128), nbox), dim3(128), 0,
+                       ctx->stream, (const double*)red, nslot, ngroups, cp->d_tri_loc,
+                       cp->d_tri_grp, cp->ntri, braw);
   PSX_CHECK_LAUNCH();
   return PSX_OK;
 }
@@ -468,7 +486,8 @@ static int contract_slots(psx_ctx* ctx, size_t lds, int* out) {
 }
 
 template <int MODE, int NLT>
-static int contract_t(psx_ctx* ctx, const ContractPlan* cp, const void* D, int N, double* braw) {
+static int contract_t(psx_ctx* ctx, const ContractPlan* cp, const void* D, int N, double* braw,
+                      const LatticeLayer* layer) {
   typedef CtTraits<MODE> Tr;
   PSX_REQUIRE(cp->maxpt == (ct_maxpt<MODE, NLT>()), "contraction plan built for another precision");
   const int64_t G = (int64_t)N * N * N;
@@ -494,7 +513,19 @@ static int contract_t(psx_ctx* ctx, const ContractPlan* cp, const void* D, int N
                cp->d_wave_mask, cp->d_wave_slot, cp->d_pair_s, pts_per_block, nslot,
                (typename Tr::TP*)part);
   PSX_CHECK_LAUNCH();
-  return launch_contract_reduce(ctx, cp, (const double*)part, nwg, ngroups, braw);
+  return launch_contract_reduce(ctx, cp, (const double*)part, nwg, ngroups, braw, 1, layer);
+}
+
+template <int MODE>
+static int contract_plan(psx_ctx* ctx, const ContractPlan* cp, const void* D, int N, double* braw,
+                         const LatticeLayer* layer = nullptr) {
+  switch (cp->nlt) {
+    case 1: return contract_t<MODE, 1>(ctx, cp, D, N, braw, layer);
+    case 2: return contract_t<MODE, 2>(ctx, cp, D, N, braw, layer);
+    case 3: return contract_t<MODE, 3>(ctx, cp, D, N, braw, layer);
+    case 4: return contract_t<MODE, 4>(ctx, cp, D, N, braw, layer);
+    default: return set_error(PSX_ERR_UNSUPPORTED, "at most 64 shells (Nmax - Ncut//step + 1 <= 64)");
+  }
 }
 
 template <int MODE>
@@ -502,13 +533,100 @@ static int contract_mode(psx_ctx* ctx, const void* D, int N, int step, int ncut,
                          double* braw) {
   const ContractPlan* cp;
   PSX_TRY(get_contract_plan(ctx, MODE, step, ncut, nmax, &cp));
-  switch (cp->nlt) {
-    case 1: return contract_t<MODE, 1>(ctx, cp, D, N, braw);
-    case 2: return contract_t<MODE, 2>(ctx, cp, D, N, braw);
-    case 3: return contract_t<MODE, 3>(ctx, cp, D, N, braw);
-    case 4: return contract_t<MODE, 4>(ctx, cp, D, N, braw);
-    default: return set_error(PSX_ERR_UNSUPPORTED, "at most 64 shells (Nmax - Ncut//step + 1 <= 64)");
+  return contract_plan<MODE>(ctx, cp, D, N, braw);
+}
+
+// A few triangles on a few shells (the aliased ones of the N^3 grid): one
+// read of the fields, every thread summing its points' products; the matrix
+// cores would run one block on one SIMD in four (measured at N = 360, two
+// triangles: see the layer's cost in psx_lattice.h).
+struct DirectTri {
+  int n;                        // triangles
+  signed char s[DIRECT_TRI][3]; // shell slots
+};
+constexpr int TD_THREADS = 256, TD_BLOCKS = 1024;
+
+__global__ __launch_bounds__(TD_THREADS) void k_tri_direct(const double* __restrict__ D, int64_t G,
+                                                           int ns, DirectTri tr,
+                                                           double* __restrict__ part) {
+  __shared__ double wsum[TD_THREADS / 64][DIRECT_TRI];
+  double acc[DIRECT_TRI];
+#pragma unroll
+  for (int t = 0; t < DIRECT_TRI; ++t) acc[t] = 0.0;
+  // two points at a time (G is a multiple of 8: N is even)
+  for (int64_t x = 2 * ((int64_t)blockIdx.x * TD_THREADS + threadIdx.x); x < G;
+       x += (int64_t)2 * TD_BLOCKS * TD_THREADS) {
+    d2v d[DIRECT_SHELLS];
+#pragma unroll
+    for (int s = 0; s < DIRECT_SHELLS; ++s) {
+      d[s][0] = d[s][1] = 0.0;
+      if (s < ns) d[s] = *reinterpret_cast<const d2v*>(D + (int64_t)s * G + x);
+    }
+#pragma unroll
+    for (int t = 0; t < DIRECT_TRI; ++t) {
+      if (t < tr.n) {
+        d2v v[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          v[k] = d[0];
+#pragma unroll
+          for (int s = 1; s < DIRECT_SHELLS; ++s)
+            if (tr.s[t][k] == s) v[k] = d[s];
+        }
+        acc[t] += v[0][0] * v[1][0] * v[2][0] + v[0][1] * v[1][1] * v[2][1];
+      }
+    }
   }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int t = 0; t < DIRECT_TRI; ++t) {
+    if (t < tr.n) {
+      double v = acc[t];
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+      if (lane == 0) wsum[wave][t] = v;
+    }
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < tr.n) {
+    double v = 0.0;
+#pragma unroll
+    for (int w = 0; w < TD_THREADS / 64; ++w) v += wsum[w][threadIdx.x];
+    part[(int64_t)blockIdx.x * DIRECT_TRI + threadIdx.x] = v;
+  }
+}
+
+// One wave per triangle: lane l adds the blocks l, l + 64, ... in order, then
+// a fixed butterfly.
+__global__ __launch_bounds__(64) void k_tri_direct_sum(const double* __restrict__ part,
+                                                       const int* __restrict__ map,
+                                                       const double* __restrict__ weight, bool add,
+                                                       double* __restrict__ braw) {
+  const int t = blockIdx.x, lane = threadIdx.x;
+  double v = 0.0;
+  for (int b = lane; b < TD_BLOCKS; b += 64) v += part[(int64_t)b * DIRECT_TRI + t];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if (lane == 0) braw[map[t]] = (add ? braw[map[t]] : 0.0) + weight[t] * v;
+}
+
+int launch_lattice_sums(psx_ctx* ctx, const void* D, const LatticeLayer& l, double* braw) {
+  if (l.cp) return contract_plan<PSX_PREC_F64>(ctx, l.cp.get(), D, l.M, braw, &l);
+  const int ns = l.nmax - l.j0 + 1;
+  PSX_REQUIRE(l.ntri <= DIRECT_TRI && ns <= DIRECT_SHELLS, "direct sums: too many triangles");
+  DirectTri tr{};
+  tr.n = l.ntri;
+  for (int t = 0; t < l.ntri; ++t)
+    for (int k = 0; k < 3; ++k) tr.s[t][k] = (signed char)(l.ijl[3 * t + k] - l.j0);
+  void* part = nullptr;
+  PSX_TRY(ctx_buffer(ctx, "direct_partials", sizeof(double) * TD_BLOCKS * DIRECT_TRI, &part));
+  hipLaunchKernelGGL(k_tri_direct, dim3(TD_BLOCKS), dim3(TD_THREADS), 0, ctx->stream,
+                     (const double*)D, (int64_t)l.M * l.M * l.M, ns, tr, (double*)part);
+  PSX_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_tri_direct_sum, dim3(l.ntri), dim3(64), 0, ctx->stream, (const double*)part,
+                     l.d_map, l.d_weight, l.add, braw);
+  PSX_CHECK_LAUNCH();
+  return PSX_OK;
 }
 
 int contract_waves_per_group(int prec, int nlt) {

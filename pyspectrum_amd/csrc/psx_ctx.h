@@ -120,6 +120,24 @@ struct ContractPlan {
   int* d_tri_ijl = nullptr;             // [ntri][3] shell indices i, j, l (reference loop order)
 };
 
+// One point set of the FP64 triangle sums (psx_lattice.h) with the triangles
+// that are summed on it.
+struct LatticeLayer {
+  int M = 0;                            // M^3 grid points
+  int j0 = 0, nmax = 0;                 // shells j0..nmax
+  bool add = false;                     // adds to the sums of an earlier layer
+  const void* phase = nullptr;          // half-cell shift: exp(-i pi k/M), k = 0..M/2, or null
+  int ntri = 0;
+  std::unique_ptr<ContractPlan> cp;     // null: the few triangles of k_tri_direct
+  std::vector<int> ijl;                 // triangles of this layer
+  int* d_map = nullptr;                 // [ntri] place in the full triangle list
+  double* d_weight = nullptr;           // [ntri] factor of the layer's sum
+};
+
+struct LatticePlan {
+  std::vector<LatticeLayer> layers;     // empty: everything on the N^3 grid
+};
+
 }  // namespace psx
 
 struct psx_ctx {
@@ -138,6 +156,7 @@ struct psx_ctx {
   std::map<int, psx::FftPlan> fft_plans;
   std::map<std::tuple<int, int, int, int, int, int>, std::unique_ptr<psx::ShellPlan>> shell_plans;
   std::map<std::tuple<int, int, int, int>, std::unique_ptr<psx::ContractPlan>> contract_plans;
+  std::map<std::tuple<int, int, int, int>, std::unique_ptr<psx::LatticePlan>> lattice_plans;
   std::map<std::string, psx::DevBuf> bufs;
   std::vector<void*> owned;  // plan allocations
   // Kernel timing (psx_ctx_kernel_timing): event pairs recorded around the
@@ -165,6 +184,8 @@ int get_contract_plan(psx_ctx* ctx, int prec, int step, int ncut, int nmax,
                       const ContractPlan** out);
 int xc_waves_per_group();
 int xc_maxpt();
+// The FP64 point sets of (N, step, ncut, nmax).
+int get_lattice_plan(psx_ctx* ctx, int N, int step, int ncut, int nmax, const LatticePlan** out);
 
 template <typename T> inline const cplx<T>* plan_tw(const FftPlan* p);
 template <> inline const cplx<float>* plan_tw<float>(const FftPlan* p) { return (const cplx<float>*)p->tw32; }
@@ -236,6 +257,12 @@ int launch_bk_finalize_batch(psx_ctx* ctx, int nbox, const double* braw, const d
 int fixed_point_exponent(double wsum_abs);
 int launch_shell_fields(psx_ctx* ctx, const void* half, int N, int step, int ncut, int nmax,
                         int prec, void* dout);
+// FP64 shell fields of a layer, [shell][M^3], from the half field of an
+// Ns^3 grid.
+int launch_lattice_fields(psx_ctx* ctx, const void* half, int Ns, int step, const LatticeLayer& l,
+                          void* dout);
+// The layer's triangle sums into (or added to) braw.
+int launch_lattice_sums(psx_ctx* ctx, const void* D, const LatticeLayer& l, double* braw);
 // z and y passes of the FP32 shell fields only (the x pass is fused into the
 // contraction): returns the plan and the intermediate T2.
 // nbox same-shape half fields back to back (box stride N*N*(N/2+1)); T2
@@ -264,6 +291,8 @@ int launch_quad_weights(psx_ctx* ctx, const float* xyz, const float* w, int64_t 
 // Fixed-order float64 reduction of contraction partials
 // [nbox][ngroups][nwg][nslot][256] and the gather of each triangle's sum
 // (reference loop order) into braw [nbox][ntri].
+// With a layer, its triangles go to their places in the full list, weighted.
 int launch_contract_reduce(psx_ctx* ctx, const ContractPlan* cp, const double* part, int64_t nwg,
-                           int ngroups, double* braw, int nbox = 1);
+                           int ngroups, double* braw, int nbox = 1,
+                           const LatticeLayer* layer = nullptr);
 }  // namespace psx

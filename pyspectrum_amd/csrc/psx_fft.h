@@ -353,5 +353,8 @@ inline void fft_stage_twiddles(const FftShape& sh, const C* full /* exp(-2 pi i 
 
 // Sizes with a compile-time instantiation; others run the runtime-N engine.
 #define PSX_FFT_SIZES(X) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(360) X(384) X(512)
+// Grid lengths of the FP64 point sets (psx_lattice.h): those and a few
+// between, so that the smallest that fits is at most a quarter too long.
+#define PSX_LAT_SIZES(X) PSX_FFT_SIZES(X) X(80) X(160) X(240) X(288) X(320)
 
 }  // namespace psx

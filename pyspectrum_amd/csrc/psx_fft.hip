@@ -167,13 +167,17 @@ __device__ __forceinline__ void store4(double* p, const double (&o)[4]) {
 }
 
 // z pass: tile (s, ky, kx0): NL kx columns of one ky row, masked to shell j.
-template <typename T, int NC>
+// LAT: the half field is that of an Ns^3 grid (the modes of the shell lie
+// inside both grids), and ph (if not null) shifts the points by half a cell:
+// mode k is multiplied by exp(-i pi (kx + ky + kz)/N), ph[n] = exp(-i pi n/N).
+template <typename T, int NC, bool LAT>
 __global__ __launch_bounds__(FFT_THREADS) void k_shell_z(const cplx<T>* __restrict__ H,
                                                          cplx<T>* __restrict__ T1,
                                                          const Tile3* __restrict__ tiles,
                                                          ShellDev sd, FftShape sh,
                                                          const cplx<T>* __restrict__ tw,
-                                                         int64_t hbs, int64_t tbs) {
+                                                         int64_t hbs, int64_t tbs, int Ns,
+                                                         const cplx<T>* __restrict__ ph) {
   // box blockIdx.y of a batch: its half field and intermediate
   H += (int64_t)blockIdx.y * hbs;
   T1 += (int64_t)blockIdx.y * tbs;
@@ -195,8 +199,12 @@ __global__ __launch_bounds__(FFT_THREADS) void k_shell_z(const cplx<T>* __restri
   const int r2 = kx * kx + kys * kys;
   const int lo = (int)min(mlo, (int64_t)1 << 30), hi = (int)min(mhi, (int64_t)1 << 30);
   const bool colin = kx < Nh;
-  const cplx<T>* src = H + (int64_t)ky * Nh + kx;
-  const int64_t rstride = (int64_t)N * Nh;
+  const cplx<T>* src = H + (int64_t)(LAT && kys < 0 ? kys + Ns : ky) * Nh + kx;
+  const int64_t rstride = (int64_t)(LAT ? Ns : N) * Nh;
+  cplx<T> pxy = mk(T(1), T(0));
+  if constexpr (LAT) {
+    if (ph && colin && r2 <= hi) pxy = ph[kx] * (kys < 0 ? conj(ph[-kys]) : ph[kys]);
+  }
   for (int nb = n0; nb < N; nb += RS * U) {
     cplx<T> v[U];
 #pragma unroll
@@ -205,7 +213,14 @@ __global__ __launch_bounds__(FFT_THREADS) void k_shell_z(const cplx<T>* __restri
       const int kzs = signed_f(n, N);
       const int m = r2 + kzs * kzs;
       v[u] = mk(T(0), T(0));
-      if (colin && n < N && m > lo && m <= hi) v[u] = src[(int64_t)n * rstride];
+      if constexpr (LAT) {
+        if (colin && n < N && m > lo && m <= hi) {
+          v[u] = src[(int64_t)(kzs < 0 ? kzs + Ns : kzs) * rstride];
+          if (ph) v[u] = v[u] * (pxy * (kzs < 0 ? conj(ph[-kzs]) : ph[kzs]));
+        }
+      } else {
+        if (colin && n < N && m > lo && m <= hi) v[u] = src[(int64_t)n * rstride];
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -348,20 +363,22 @@ __global__ __launch_bounds__(FFT_THREADS) void k_shell_x(const cplx<T>* __restri
   }
 }
 
-template <typename T, int NC>
+// LAT: the half field H is that of an Ns^3 grid, shifted by the phases ph.
+template <typename T, int NC, bool LAT = false>
 static int shell_fields_n(psx_ctx* ctx, const FftPlan* p, const ShellPlan* sp, const cplx<T>* H,
                           int step, cplx<T>* t1, cplx<T>* t2, T* dout, bool do_x = true,
-                          int nbox = 1) {
+                          int nbox = 1, int Ns = 0, const cplx<T>* ph = nullptr) {
   const int64_t hbs = (int64_t)p->shape.N * p->shape.N * (p->shape.N / 2 + 1);
   const int N = p->shape.N;
-  ShellDev sd{sp->d_meta, sp->d_off, step, N / 2 + 1};
+  ShellDev sd{sp->d_meta, sp->d_off, step, (LAT ? Ns : N) / 2 + 1};
   const size_t ldsz = ((size_t)TileCfg<T>::LINES * (N + 1) + N) * sizeof(cplx<T>);
   const size_t ldsx = ((size_t)shell_x_pairs<T>(NC) * (N + PSX_XPAD) + N) * sizeof(cplx<T>);
   const cplx<T>* tw = plan_tw<T>(p);
   if (sp->nz_tiles > 0) {
-    PSX_TRY(set_lds(k_shell_z<T, NC>, ldsz));
-    launch_timed(ctx, "k_shell_z", k_shell_z<T, NC>, dim3(sp->nz_tiles, nbox), dim3(FFT_THREADS),
-                 ldsz, H, t1, sp->d_ztiles, sd, p->shape, tw, hbs, sp->t_elems);
+    auto kern = k_shell_z<T, NC, LAT>;
+    PSX_TRY(set_lds(kern, ldsz));
+    launch_timed(ctx, "k_shell_z", kern, dim3(sp->nz_tiles, nbox), dim3(FFT_THREADS), ldsz, H, t1,
+                 sp->d_ztiles, sd, p->shape, tw, hbs, sp->t_elems, Ns, ph);
     PSX_CHECK_LAUNCH();
   }
   if (sp->ny_tiles > 0) {
@@ -403,6 +420,34 @@ static int shell_fields_t(psx_ctx* ctx, const cplx<T>* H, int N, int step, int n
   switch (N) {
     PSX_FFT_SIZES(PSX_CASE_N)
     default: return shell_fields_n<T, 0>(ctx, p, sp, H, step, (cplx<T>*)t1, (cplx<T>*)t2, (T*)dout);
+  }
+}
+#undef PSX_CASE_N
+
+// FP64 shell fields on a layer's M^3 points (M from PSX_LAT_SIZES) or, for
+// the layer of the source grid itself (M = Ns), the general path.
+#define PSX_CASE_N(n)                                                                          \
+  case n:                                                                                      \
+    return shell_fields_n<double, n, true>(ctx, p, sp, (const cplx<double>*)half, step,        \
+                                           (cplx<double>*)t1, (cplx<double>*)t2, (double*)dout, \
+                                           true, 1, Ns, (const cplx<double>*)l.phase);
+
+int launch_lattice_fields(psx_ctx* ctx, const void* half, int Ns, int step, const LatticeLayer& l,
+                          void* dout) {
+  if (l.M == Ns)
+    return shell_fields_t<double>(ctx, (const cplx<double>*)half, Ns, step, l.j0 * step, l.nmax,
+                                  dout);
+  const FftPlan* p;
+  PSX_TRY(get_fft_plan(ctx, l.M, &p));
+  const ShellPlan* sp;
+  PSX_TRY(get_shell_plan(ctx, l.M, step, l.j0 * step, l.nmax, TileCfg<double>::LINES,
+                         PSX_SHELL_X_PAIRS_F64, &sp));
+  void *t1 = nullptr, *t2 = nullptr;
+  PSX_TRY(ctx_buffer(ctx, "shell_t1_f64", (size_t)sp->t_elems * sizeof(cplx<double>), &t1));
+  PSX_TRY(ctx_buffer(ctx, "shell_t2_f64", (size_t)sp->t_elems * sizeof(cplx<double>), &t2));
+  switch (l.M) {
+    PSX_LAT_SIZES(PSX_CASE_N)
+    default: return set_error(PSX_ERR_UNSUPPORTED, "layer size without an FFT instantiation");
   }
 }
 #undef PSX_CASE_N

@@ -4,6 +4,9 @@
 #pragma once
 #include <algorithm>
 #include <cstdint>
+#include <map>
+#include <numeric>
+#include <utility>
 #include <vector>
 
 namespace psx {
@@ -172,6 +175,224 @@ inline void triangle_cover(const std::vector<int>& ijl, int nmax, int j0, std::v
       }
     }
   }
+}
+
+// ---------------------------------------------------- contract layout ----
+// What the contraction kernel needs to know of the plan: its wave layout.
+struct LayoutShape {
+  bool f64 = false;           // float64 MFMA output layout, no LDS bank arrangement
+  bool simd_balance = false;  // one workgroup per CU: balance the four SIMDs
+  int maxpt = 0, wpg = 0;     // pair tiles per wave, waves per workgroup
+};
+
+struct ContractLayout {
+  int npairs = 0, npt = 0, nblk = 0, waves = 0, nslot = 0;
+  std::vector<int> wave_pt, wave_mask, wave_slot, pair_s, tri_loc, tri_grp;
+};
+
+// Split-BF16 contraction: the LDS serves the 16-byte A reads of 8 rows of a
+// pair tile per cycle, conflict-free when their distinct shells differ
+// modulo 8 (float rows 8 words apart modulo 64 banks).  Swap rows between
+// the two 8-row halves of each tile while that lowers the number of shells
+// that share a bank group with another shell of their half (i and j
+// columns).  Row order inside a tile does not change any result.
+inline void arrange_half_tiles(std::vector<int>* prow, int nsh, int j0) {
+  auto half_cost = [&](const int* r) {
+    int c = 0;
+    for (int col = 0; col < 2; ++col) {
+      int seen[64], nseen = 0, grp[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      for (int k = 0; k < 8; ++k) {
+        if (r[k] < 0) continue;
+        const int sh = (col == 0 ? r[k] / nsh : r[k] % nsh) - j0;
+        bool dup = false;
+        for (int m = 0; m < nseen; ++m) dup |= seen[m] == sh;
+        if (dup) continue;
+        seen[nseen++] = sh;
+        c += grp[sh & 7]++ > 0 ? 1 : 0;
+      }
+    }
+    return c;
+  };
+  for (size_t t = 0; t + 16 <= prow->size(); t += 16) {
+    int* r = prow->data() + t;
+    int cur = half_cost(r) + half_cost(r + 8);
+    for (bool improved = true; improved;) {
+      improved = false;
+      for (int a = 0; a < 8; ++a)
+        for (int b = 8; b < 16; ++b) {
+          std::swap(r[a], r[b]);
+          const int c2 = half_cost(r) + half_cost(r + 8);
+          if (c2 < cur) { cur = c2; improved = true; }
+          else std::swap(r[a], r[b]);
+        }
+    }
+  }
+}
+
+// Pair tiles, their assignment to waves and the place of every triangle's sum
+// for the triangles ijl on the shells j0..nmax.  False if a triangle has no
+// chosen pair.
+inline bool contract_layout(const std::vector<int>& ijl, int j0, int nmax, const LayoutShape& ls,
+                            ContractLayout* cl) {
+  const int ntri = (int)(ijl.size() / 3);
+  std::vector<int> tpair, tshell;
+  triangle_cover(ijl, nmax, j0, &tpair, &tshell);
+  for (int t = 0; t < ntri; ++t)
+    if (tpair[t] < 0) return false;
+  // pair tiles: pairs grouped by their set of column tiles, whole tiles of one
+  // set first, the remainders sorted by (tiles used, set) and cut into tiles
+  std::map<int, int> pmask;  // pair key -> column tiles it reads
+  for (int t = 0; t < ntri; ++t) pmask[tpair[t]] |= 1 << ((tshell[t] - j0) / 16);
+  std::map<int, std::vector<int>> by_mask;
+  for (const auto& pm : pmask) by_mask[pm.second].push_back(pm.first);
+  std::vector<int> prow;  // pair key of each row, -1 = padding
+  std::vector<std::pair<int, int>> rest;
+  for (const auto& bm : by_mask) {
+    const size_t whole = bm.second.size() / 16 * 16;
+    prow.insert(prow.end(), bm.second.begin(), bm.second.begin() + whole);
+    for (size_t k = whole; k < bm.second.size(); ++k) rest.push_back({bm.first, bm.second[k]});
+  }
+  std::stable_sort(rest.begin(), rest.end(), [](const std::pair<int, int>& a, const std::pair<int, int>& b) {
+    const int pa = __builtin_popcount(a.first), pb = __builtin_popcount(b.first);
+    return pa != pb ? pa < pb : a.first < b.first;
+  });
+  for (const auto& r : rest) prow.push_back(r.second);
+  cl->npairs = (int)prow.size();
+  cl->npt = (cl->npairs + 15) / 16;
+  prow.resize((size_t)cl->npt * 16, -1);
+  const int nsh = nmax + 1;
+  if (!ls.f64) arrange_half_tiles(&prow, nsh, j0);
+  std::vector<int>& pair_s = cl->pair_s;
+  pair_s.assign(2 * prow.size(), -1);
+  std::map<int, int> prow_of;
+  for (size_t r = 0; r < prow.size(); ++r) {
+    if (prow[r] < 0) continue;
+    pair_s[2 * r] = prow[r] / nsh - j0;
+    pair_s[2 * r + 1] = prow[r] % nsh - j0;
+    prow_of[prow[r]] = (int)r;
+  }
+  std::vector<int> ptmask(cl->npt, 0);
+  std::vector<int> tpt(ntri), trow(ntri), tlt(ntri), tcol(ntri);
+  for (int t = 0; t < ntri; ++t) {
+    const int p = prow_of.at(tpair[t]);
+    tpt[t] = p / 16; trow[t] = p % 16;
+    tlt[t] = (tshell[t] - j0) / 16; tcol[t] = (tshell[t] - j0) % 16;
+    ptmask[tpt[t]] |= 1 << tlt[t];
+  }
+  cl->nblk = 0;
+  for (int m : ptmask) cl->nblk += __builtin_popcount(m);
+  // assign pair tiles to waves: groups of WPG waves x maxpt slots, greedy by load
+  const int maxpt = ls.maxpt, WPG = ls.wpg;
+  const int ngroups = (cl->npt + WPG * maxpt - 1) / (WPG * maxpt);
+  const int nw = ngroups * WPG;
+  std::vector<int> order(cl->npt);
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+    return __builtin_popcount(ptmask[a]) > __builtin_popcount(ptmask[b]);
+  });
+  std::vector<int> load(nw, 0), cnt(nw, 0);
+  std::vector<int>&wave_pt = cl->wave_pt, &wave_mask = cl->wave_mask;
+  wave_pt.assign(nw * maxpt, -1);
+  wave_mask.assign(nw * maxpt, 0);
+  std::vector<int> pt_wave(cl->npt), pt_q(cl->npt);
+  for (int pt : order) {
+    int best = -1;
+    for (int w = 0; w < nw; ++w)
+      if (cnt[w] < maxpt && (best < 0 || load[w] < load[best])) best = w;
+    wave_pt[best * maxpt + cnt[best]] = pt;
+    wave_mask[best * maxpt + cnt[best]] = ptmask[pt];
+    pt_wave[pt] = best; pt_q[pt] = cnt[best];
+    cnt[best]++;
+    // cost of a tile: forming and splitting its products (about three
+    // blocks' worth of MFMA time) plus its output blocks
+    load[best] += 3 + __builtin_popcount(ptmask[pt]);
+  }
+  // Fused layout (one workgroup per CU): the waves of the workgroup are
+  // spread over the CU's four SIMDs (wave w on SIMD w % 4), and a SIMD issues
+  // its waves' VALU and MFMA work one at a time, so what bounds the group is
+  // the busiest SIMD.  Swap tiles (or a tile and an empty slot) between waves
+  // of different SIMDs while that lowers the group's (largest SIMD load, sum
+  // of squared SIMD loads).  Which wave runs a tile changes no result: its
+  // sums are formed in the same order.  (Measured at Ngrid 360, 40 shells:
+  // k_xcontract 6.13 -> 5.95 ms; the staged k_contract, several workgroups
+  // per CU, ran 4-6 % slower with it and keeps the per-wave balance.)
+  if (ls.simd_balance && WPG % 4 == 0) {
+    auto tcost = [&](int pt) { return pt < 0 ? 0 : 3 + __builtin_popcount(ptmask[pt]); };
+    for (int g = 0; g < ngroups; ++g) {
+      const int w0 = g * WPG;
+      auto score = [&](long long* sq) {
+        int sl[4] = {0, 0, 0, 0};
+        for (int w = w0; w < w0 + WPG; ++w) sl[(w - w0) % 4] += load[w];
+        *sq = 0;
+        int mx = 0;
+        for (int s = 0; s < 4; ++s) { mx = std::max(mx, sl[s]); *sq += (long long)sl[s] * sl[s]; }
+        return mx;
+      };
+      long long sq;
+      int mx = score(&sq);
+      for (bool improved = true; improved;) {
+        improved = false;
+        for (int a = w0 * maxpt; a < (w0 + WPG) * maxpt; ++a)
+          for (int b = a + 1; b < (w0 + WPG) * maxpt; ++b) {
+            const int wa = a / maxpt, wb = b / maxpt;
+            if ((wa - w0) % 4 == (wb - w0) % 4 || wave_pt[a] == wave_pt[b]) continue;
+            const int d = tcost(wave_pt[b]) - tcost(wave_pt[a]);
+            load[wa] += d; load[wb] -= d;
+            long long sq2;
+            const int mx2 = score(&sq2);
+            if (mx2 < mx || (mx2 == mx && sq2 < sq)) {
+              std::swap(wave_pt[a], wave_pt[b]);
+              std::swap(wave_mask[a], wave_mask[b]);
+              mx = mx2; sq = sq2; improved = true;
+            } else {
+              load[wa] -= d; load[wb] += d;
+            }
+          }
+      }
+    }
+    // slots in use first within each wave (the kernels count a wave's tiles)
+    for (int w = 0; w < nw; ++w)
+      for (int q = 0; q < maxpt; ++q)
+        for (int r = q + 1; r < maxpt && wave_pt[w * maxpt + q] < 0; ++r)
+          if (wave_pt[w * maxpt + r] >= 0) {
+            std::swap(wave_pt[w * maxpt + q], wave_pt[w * maxpt + r]);
+            std::swap(wave_mask[w * maxpt + q], wave_mask[w * maxpt + r]);
+          }
+    for (int w = 0; w < nw; ++w)
+      for (int q = 0; q < maxpt; ++q) {
+        const int pt = wave_pt[w * maxpt + q];
+        if (pt >= 0) { pt_wave[pt] = w; pt_q[pt] = q; }
+      }
+  }
+  // output slots per group: the blocks that hold a triangle
+  std::vector<int>& wave_slot = cl->wave_slot;
+  wave_slot.assign(nw * maxpt * 4, -1);
+  std::vector<int> gslots(ngroups, 0);
+  for (int w = 0; w < nw; ++w)
+    for (int q = 0; q < maxpt; ++q) {
+      const int pt = wave_pt[w * maxpt + q];
+      for (int t = 0; t < 4; ++t)
+        if (pt >= 0 && ((ptmask[pt] >> t) & 1)) wave_slot[(w * maxpt + q) * 4 + t] = gslots[w / WPG]++;
+    }
+  cl->nslot = *std::max_element(gslots.begin(), gslots.end());
+  std::vector<int>&tri_loc = cl->tri_loc, &tri_grp = cl->tri_grp;
+  tri_loc.assign(ntri, 0);
+  tri_grp.assign(ntri, 0);
+  for (int t = 0; t < ntri; ++t) {
+    const int w = pt_wave[tpt[t]], q = pt_q[tpt[t]];
+    const int slot = wave_slot[(w * maxpt + q) * 4 + tlt[t]];
+    const int row = trow[t], col = tcol[t];
+    // 16x16 MFMA output layout (measured on gfx950): f32 outputs (f32 and bf16
+    // inputs) hold row r in lane col + 16*(r/4), register r%4; the f64 MFMA
+    // holds it in lane col + 16*(r%4), register r/4.
+    const bool f64 = ls.f64;
+    const int lane = col + 16 * (f64 ? row % 4 : row / 4);
+    const int reg = f64 ? row / 4 : row % 4;
+    tri_loc[t] = slot * 256 + lane * 4 + reg;
+    tri_grp[t] = w / WPG;
+  }
+  cl->waves = nw;
+  return true;
 }
 
 }  // namespace psx
