@@ -259,6 +259,7 @@ static int build_contract_plan(psx_ctx* ctx, int prec, bool fused, const std::ve
   LayoutShape ls;
   ls.f64 = prec == PSX_PREC_F64;
   ls.simd_balance = fused;
+  ls.mfma_bound = prec != PSX_PREC_BF16X3;
   ls.maxpt = fused ? xc_maxpt() : contract_maxpt(prec, nlt);
   ls.wpg = fused ? xc_waves_per_group() : contract_waves_per_group(prec, nlt);
   ContractLayout cl;

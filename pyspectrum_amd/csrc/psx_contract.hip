@@ -75,14 +75,14 @@ constexpr int CT_MAXLT = 4;   // l tiles in the plan layout (ns <= 64)
 template <int MODE> struct CtTraits;
 template <> struct CtTraits<PSX_PREC_F64> {
   typedef double TD; typedef d4v Acc; typedef double TP;
-  static constexpr int KC = 128, MAXPT = 4, PAD = 2;
+  static constexpr int KC = 128, MAXPT = 4, PAD = 2, QPAD = 16;
 };
 #ifndef PSX_CT_KC_F32
 #define PSX_CT_KC_F32 128
 #endif
 template <> struct CtTraits<PSX_PREC_F32> {
   typedef float TD; typedef f4v Acc; typedef double TP;
-  static constexpr int KC = PSX_CT_KC_F32, MAXPT = 2, PAD = 4;
+  static constexpr int KC = PSX_CT_KC_F32, MAXPT = 2, PAD = 4, QPAD = 0;
 };
 #ifndef PSX_CT_PAD_BF
 #define PSX_CT_PAD_BF 8     // float rows: 264 words = 8 modulo 64 banks
@@ -92,7 +92,7 @@ template <> struct CtTraits<PSX_PREC_F32> {
 #endif
 template <> struct CtTraits<PSX_PREC_BF16X3> {
   typedef float TD; typedef f4v Acc; typedef double TP;
-  static constexpr int KC = PSX_CT_KC_BF, MAXPT = 3, PAD = PSX_CT_PAD_BF;
+  static constexpr int KC = PSX_CT_KC_BF, MAXPT = 3, PAD = PSX_CT_PAD_BF, QPAD = 0;
 };
 
 // Waves per workgroup and pair tiles per wave.  Split-BF16 up to 3 l tiles:
@@ -121,8 +121,11 @@ template <int MODE, int NLT> __host__ __device__ constexpr int ct_maxpt() {
 template <int MODE, int NLT> __host__ __device__ constexpr int ct_kc() {
   return (MODE == PSX_PREC_BF16X3 && NLT > 3) ? PSX_CT_KC_BF4 : CtTraits<MODE>::KC;
 }
+// QPAD: elements between the quarters of a row (FP64: the lane groups read
+// 32 words modulo 64 banks apart instead of all from the same banks; 10.24 ->
+// 10.0 ms on the layers of N = 360, 40 shells).
 template <int MODE, int NLT> __host__ __device__ constexpr int ct_ldw() {
-  return ct_kc<MODE, NLT>() + CtTraits<MODE>::PAD;
+  return ct_kc<MODE, NLT>() + 4 * CtTraits<MODE>::QPAD + CtTraits<MODE>::PAD;
 }
 template <int MODE, int NLT> __host__ __device__ constexpr int ct_ldwh() {
   return ct_kc<MODE, NLT>() + PSX_CT_PADH_BF;
@@ -152,6 +155,7 @@ __global__ __launch_bounds__((ct_waves<MODE, NLT>() * 64), PSX_CT_MINW) void k_c
   constexpr int LDWH = ct_ldwh<MODE, NLT>();
   constexpr bool BF = MODE == PSX_PREC_BF16X3;
   constexpr int KQ = KC / 4;  // F32/F64: points per lane group per chunk
+  constexpr int QS = KQ + Tr::QPAD;  // and where the next group's begin
   extern __shared__ __align__(16) unsigned char smem_raw[];
   TD* lds = reinterpret_cast<TD*>(smem_raw);
   unsigned short* ldh = reinterpret_cast<unsigned short*>(smem_raw + (size_t)(ns + 1) * LDW * sizeof(TD));
@@ -169,7 +173,7 @@ __global__ __launch_bounds__((ct_waves<MODE, NLT>() * 64), PSX_CT_MINW) void k_c
   const int r16 = lane & 15;   // row (A) / column (B) within a 16-block
   const int kq = lane >> 4;    // k group
   const int gw = (int)blockIdx.y * CT_WAVES + wave;
-  const int kbase = BF ? kq * 4 : kq * KQ;   // float rows
+  const int kbase = BF ? kq * 4 : kq * QS;   // float rows
   const int kbaseh = kq * 8;                  // bf16 planes (split-BF16)
   // bf16 pairs (lo, hi) = (-1, 0) and (0, -1) for the split residuals
   const unsigned neg_lo = in_register(0x0000BF80u), neg_hi = in_register(0xBF800000u);
@@ -260,8 +264,9 @@ __global__ __launch_bounds__((ct_waves<MODE, NLT>() * 64), PSX_CT_MINW) void k_c
         } else {
           d2v v0, v1;
           v0[0] = pre[u][0]; v0[1] = pre[u][1]; v1[0] = pre[u][2]; v1[1] = pre[u][3];
-          *reinterpret_cast<d2v*>(lds + s * LDW + k) = v0;
-          *reinterpret_cast<d2v*>(lds + s * LDW + k + 2) = v1;
+          TD* dst = lds + s * LDW + k / KQ * Tr::QPAD + k;
+          *reinterpret_cast<d2v*>(dst) = v0;
+          *reinterpret_cast<d2v*>(dst + 2) = v1;
         }
         if constexpr (BF) {
           // x = hi + lo, hi = bf16(x), lo = bf16(x - hi) (x - hi is exact)

@@ -180,8 +180,9 @@ inline void triangle_cover(const std::vector<int>& ijl, int nmax, int j0, std::v
 // ---------------------------------------------------- contract layout ----
 // What the contraction kernel needs to know of the plan: its wave layout.
 struct LayoutShape {
-  bool f64 = false;           // float64 MFMA output layout, no LDS bank arrangement
+  bool f64 = false;           // float64 MFMA output layout
   bool simd_balance = false;  // one workgroup per CU: balance the four SIMDs
+  bool mfma_bound = false;    // the blocks' MFMAs, not the products, take the time
   int maxpt = 0, wpg = 0;     // pair tiles per wave, waves per workgroup
 };
 
@@ -261,7 +262,7 @@ inline bool contract_layout(const std::vector<int>& ijl, int j0, int nmax, const
   cl->npt = (cl->npairs + 15) / 16;
   prow.resize((size_t)cl->npt * 16, -1);
   const int nsh = nmax + 1;
-  if (!ls.f64) arrange_half_tiles(&prow, nsh, j0);
+  arrange_half_tiles(&prow, nsh, j0);
   std::vector<int>& pair_s = cl->pair_s;
   pair_s.assign(2 * prow.size(), -1);
   std::map<int, int> prow_of;
@@ -297,15 +298,30 @@ inline bool contract_layout(const std::vector<int>& ijl, int j0, int nmax, const
   std::vector<int> pt_wave(cl->npt), pt_q(cl->npt);
   for (int pt : order) {
     int best = -1;
-    for (int w = 0; w < nw; ++w)
-      if (cnt[w] < maxpt && (best < 0 || load[w] < load[best])) best = w;
+    if (ls.mfma_bound) {
+      // F32/F64: a block's MFMAs take 8 to 16 times as long as a tile's
+      // products, so the four SIMDs (wave w on SIMD w % 4) share the blocks:
+      // the least loaded SIMD of a group that has room, then its least
+      // loaded wave (46 blocks: at most 12 on a SIMD instead of 13; 40 shells
+      // at N = 360: FP32 10.15 -> 9.67 ms, the FP64 layers 10.0 -> 9.3 ms)
+      std::vector<int> sl(ngroups * 4, 0);
+      for (int w = 0; w < nw; ++w) sl[w / WPG * 4 + w % WPG % 4] += load[w];
+      auto simd = [&](int w) { return sl[w / WPG * 4 + w % WPG % 4]; };
+      for (int w = 0; w < nw; ++w)
+        if (cnt[w] < maxpt && (best < 0 || simd(w) < simd(best) ||
+                               (simd(w) == simd(best) && load[w] < load[best])))
+          best = w;
+    } else {
+      for (int w = 0; w < nw; ++w)
+        if (cnt[w] < maxpt && (best < 0 || load[w] < load[best])) best = w;
+    }
     wave_pt[best * maxpt + cnt[best]] = pt;
     wave_mask[best * maxpt + cnt[best]] = ptmask[pt];
     pt_wave[pt] = best; pt_q[pt] = cnt[best];
     cnt[best]++;
     // cost of a tile: forming and splitting its products (about three
     // blocks' worth of MFMA time) plus its output blocks
-    load[best] += 3 + __builtin_popcount(ptmask[pt]);
+    load[best] += (ls.mfma_bound ? 1 : 3) + (ls.mfma_bound ? 8 : 1) * __builtin_popcount(ptmask[pt]);
   }
   // Fused layout (one workgroup per CU): the waves of the workgroup are
   // spread over the CU's four SIMDs (wave w on SIMD w % 4), and a SIMD issues
