@@ -581,6 +581,27 @@ __device__ __forceinline__ void fcomb_iteration(cplx<T> (&m)[8], const FcombSlot
   slot_put(m, sl.canon(1, 1, 1), conj(slot_get(m, sl.canon(0, 0, 0))));
 }
 
+// The value that iteration leaves at (ix, +-iy, +-iz) (*q = 2 yb + zb) as one
+// of its combinations c000, c001, c010, c011 (*q on return) or the conjugate
+// of one (*cj): stores 0..3 put c_q, store p >= 4 the conjugate of what slot
+// (0, 7 - p) then holds; the last store into a slot decides.
+__device__ __forceinline__ void fcomb_survivor(const FcombSlots& sl, int* q, bool* cj) {
+  int slot = sl.canon(0, *q >> 1, *q & 1), before = 8;
+  bool conjugate = false;
+  for (;;) {
+    int p = before - 1;
+    while (sl.canon(p >> 2, (p >> 1) & 1, p & 1) != slot) --p;  // its own store 0..3 at the latest
+    if (p < 4) {
+      *q = p;
+      *cj = conjugate;
+      return;
+    }
+    slot = sl.canon(0, ((7 - p) >> 1) & 1, (7 - p) & 1);
+    before = p;
+    conjugate = !conjugate;
+  }
+}
+
 // Box blockIdx.y of a batch: grid F [box][N^3], half field Hh [box][N^2 (N/2+1)].
 template <typename T>
 __global__ __launch_bounds__(256) void k_fcomb(const cplx<T>* __restrict__ F, cplx<T>* __restrict__ Hh, int N,
@@ -625,6 +646,19 @@ __global__ __launch_bounds__(256) void k_fcomb(const cplx<T>* __restrict__ F, cp
 // (where x, y or z alias, the other lines of the iteration coincide with
 // these two).  A tile holds tp such line pairs, consecutive x at one y; the
 // line transforms are those of k_fft_lines, the combination that of k_fcomb.
+//
+//
+// The lines fill the LDS (two or three workgroups a CU), so between loads and
+// stores the kernel is bound by its own instructions and latencies.  A thread
+// stays on one line of the loads and on one pair of the epilogue: addresses
+// are a base plus a constant stride and the x and y factors of the twiddle and
+// the window are formed once (no index divisions, a third of the float64
+// products), and nothing is kept in scratch memory.  Measured (float): N = 360
+// 0.288 -> 0.254 ms, 16 boxes of 128 0.193 -> 0.127, 300 (runtime N) 0.52 ->
+// 0.235, 512 0.98 -> 0.95; reading the grid and writing the half field once
+// takes 0.12, 0.09, 0.07 and 0.33 at 4.8 TB/s.  (Several tiles a workgroup with
+// the next one's elements loaded ahead into registers: 512 0.83, but 0.151 for
+// the 16 boxes and 0.25 -> 0.25 at 360, where the registers cost a workgroup.)
 template <typename T, int NC>
 __global__ __launch_bounds__(FFT_THREADS) void k_fft_zcomb(const cplx<T>* __restrict__ F,
                                                             cplx<T>* __restrict__ Hh, FftShape sh,
@@ -646,68 +680,68 @@ __global__ __launch_bounds__(FFT_THREADS) void k_fft_zcomb(const cplx<T>* __rest
   const int ntx = (Nh + tp - 1) / tp;
   // neighbouring x tiles read the two halves of the same 128-byte lines
   const int bx = xcd_local_block((int)blockIdx.x, (int)gridDim.x);
-  const int y = bx / ntx;
-  const int x0 = (bx - y * ntx) * tp;
-  const int np = min(tp, Nh - x0);
-  const int yb_line = (N - y) % N;
-  // line 2c: (x0 + c, y); line 2c + 1: (-(x0 + c), -y); element n along z
-  batched_fill<8, cplx<T>>(
-      2 * tp * N,
-      [&](int idx) {
-        const int n = idx / (2 * tp), l = idx - n * (2 * tp);
-        const int c = l >> 1;
-        if (c >= np) return mk(T(0), T(0));
-        const int x = (l & 1) ? (N - (x0 + c)) % N : x0 + c;
-        const int yy = (l & 1) ? yb_line : y;
-        return F[((int64_t)n * N + yy) * N + x];
-      },
-      [&](int idx, cplx<T> v) {
-        const int n = idx / (2 * tp), l = idx - n * (2 * tp);
-        if ((l >> 1) < np) lds[l * lstride + n] = v;
-      });
+  const int y = bx / ntx, x0 = (bx - y * ntx) * tp, np = min(tp, Nh - x0);
+  // line 2c: (x0 + c, y); line 2c + 1: (-(x0 + c), -y); element n along z: rows
+  // n0, n0 + RS, ... of one line, U loads in flight
+  {
+    constexpr int U = 8;
+    const int nl = 2 * tp, RS = FFT_THREADS / nl;
+    const int n0 = (int)threadIdx.x / nl, l = (int)threadIdx.x - n0 * nl, c = l >> 1;
+    if (n0 < RS && c < np) {
+      const int xc = x0 + c;
+      const int x = (l & 1) && xc > 0 ? N - xc : xc, ym = y > 0 ? N - y : 0;
+      const cplx<T>* src = F + (int64_t)((l & 1) ? ym : y) * N + x;
+      cplx<T>* dst = lds + l * lstride;
+      for (int nb = n0; nb < N; nb += RS * U) {
+        cplx<T> v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = src[(int64_t)min(nb + u * RS, N - 1) * NN];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (nb + u * RS < N) dst[nb + u * RS] = v[u];
+      }
+    }
+  }
   cplx<T>* twl = lds + tl * lstride;
   stage_twiddles(twl, tw, N);
   __syncthreads();
   fft_tile<NC, 1, T, ML, TileCfg<T>::ELEMS>(lds, sh, 2 * np, lstride, twl);
-  const int yb = y > N / 2 ? 1 : 0, iy = yb ? N - y : y;
-  for (int idx = threadIdx.x; idx < np * N; idx += FFT_THREADS) {
-    const int z = idx / np, c = idx - z * np;
-    const int ix = x0 + c;
-    const int zb = z > N / 2 ? 1 : 0, iz = zb ? N - z : z;
-    const int xs[2] = {ix, (N - ix) % N};
-    const int ys[2] = {iy, (N - iy) % N};
-    const int zs[2] = {iz, (N - iz) % N};
-    const FcombSlots sl{xs[0] == xs[1], ys[0] == ys[1], zs[0] == zs[1]};
-    const cplx<T>* la = lds + (2 * c) * lstride;      // (ix, y)
-    const cplx<T>* lb = lds + (2 * c + 1) * lstride;  // (-ix, -y)
-    cplx<T> out;
-    if (!(sl.ax || sl.ay || sl.az)) {
-      // no index aliases: the element keeps its own combination c_{0,yb,zb}
-      // = v (1 - t) + conj(v') (1 + t) times cfac, v = F(k), v' = F(-k), with
-      // the twiddle t of k_fcomb's cma/cmb/cmc/cmd (the same operations)
-      const c64 xr = rec[ix], yr = rec[iy], zr = rec[iz];
-      const c64 ixr = mk(-xr.im, xr.re);
-      const c64 yv = yb ? conj(yr) : yr;
-      c64 t64;
-      if (yb && zb) t64 = ixr * conj(yr * zr);
-      else t64 = ixr * yv * (zb ? conj(zr) : zr);
-      const cplx<T> t = mk((T)t64.re, (T)t64.im);
-      const cplx<T> one = mk(T(1), T(0));
-      const T cfac = cf / (window_val<T>(Wf, Wd, ix) * window_val<T>(Wf, Wd, iy) *
-                           window_val<T>(Wf, Wd, iz));
-      out = (la[z] * (one - t) + conj(lb[(N - z) % N]) * (one + t)) * cfac;
-    } else {
-      cplx<T> m[8];
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const int X = xs[s >> 2], Y = ys[(s >> 1) & 1], Z = zs[s & 1];
-        // every (X, Y) the iteration needs here is one of the two lines
-        m[s] = (X == ix && Y == y) ? la[Z] : lb[Z];
-      }
-      fcomb_iteration(m, sl, ix, iy, iz, cf, rec, Wf, Wd);
-      out = slot_get(m, sl.canon(0, yb, zb));
-    }
-    Hh[((int64_t)z * N + y) * Nh + ix] = out;
+  // epilogue: pair c, rows z0, z0 + RZ, ...
+  const int RZ = FFT_THREADS / tp;
+  const int zfirst = (int)threadIdx.x / tp, c = (int)threadIdx.x - zfirst * tp;
+  if (zfirst >= RZ || c >= np) return;
+  const int yb = y > N / 2 ? 1 : 0, iy = yb ? N - y : y, ix = x0 + c;
+  const c64 xr = rec[ix], yr = rec[iy];
+  const c64 ixr = mk(-xr.im, xr.re);
+  const c64 ixy0 = ixr * yr, ixy1 = ixr * conj(yr);
+  const T wxy = window_val<T>(Wf, Wd, ix) * window_val<T>(Wf, Wd, iy);
+  const cplx<T> one = mk(T(1), T(0));
+  const cplx<T>* la = lds + (2 * c) * lstride;      // (ix, y)
+  const cplx<T>* lb = lds + (2 * c + 1) * lstride;  // (-ix, -y)
+  cplx<T>* dst = Hh + (int64_t)y * Nh + ix;
+  const bool ax = ix == 0 || 2 * ix == N, ay = iy == 0 || 2 * iy == N;
+  for (int z = zfirst; z < N; z += RZ) {
+    const int zb = z > N / 2 ? 1 : 0, iz = zb ? N - z : z, mz = z > 0 ? N - z : 0;
+    // The element is the combination c_q (q = 2 yb + zb) of its iteration,
+    // or, where an index aliases, the one whose store survives there (cj:
+    // conjugated).
+    int q = 2 * yb + zb;
+    bool cj = false;
+    if (ax || ay || z == mz) fcomb_survivor(FcombSlots{ax, ay, z == mz}, &q, &cj);
+    const bool yq = (q & 2) != 0, zq = (q & 1) != 0;
+    // c_q = v (1 - t) + conj(v') (1 + t) times cfac, v at (ix, +-iy, +-iz)
+    // by q and v' its mirror; both lie on the two lines.  The twiddle t in
+    // double (estimator.f:650-653), rounded to T.
+    const c64 zr = rec[iz];
+    const c64 t64 = q == 3 ? ixr * conj(yr * zr) : (yq ? ixy1 : ixy0) * (zq ? conj(zr) : zr);
+    const cplx<T> t = mk((T)t64.re, (T)t64.im);
+    const T cfac = cf / (wxy * window_val<T>(Wf, Wd, iz));
+    const bool same_y = yq == (yb != 0), same_z = zq == (zb != 0);
+    const cplx<T> va = (ay || same_y ? la : lb)[same_z ? z : mz];
+    const cplx<T> vm = (ax && (ay || !same_y) ? la : lb)[same_z ? mz : z];
+    cplx<T> out = (va * (one - t) + conj(vm) * (one + t)) * cfac;
+    if (cj) out = conj(out);
+    dst[(int64_t)z * N * Nh] = out;
   }
 }
 
