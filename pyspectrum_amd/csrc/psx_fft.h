@@ -14,11 +14,12 @@
 // Stage order: odd radices first (their stride-R scatter in the first stage
 // touches every LDS bank once per 16 lanes), then 4/2, then the 8s.
 //
-// Two instantiations of the same stage code:
+// Two instantiations:
 //  * compile-time N (template parameter, the sizes the estimator uses): the
 //    radix sequence, butterfly counts and all index divisions are constants,
 //    and per-thread register arrays are sized exactly;
-//  * runtime N (N = 0): any supported size, used for the others.
+//  * runtime N (N = 0): any supported size, used for the others, with one wave
+//    per line instead of the mapping above.
 //
 // Twiddles: one table of N entries per N, stage after stage, row k of a
 // stage holding exp(-2 pi i r k / (Ns R)) for r = 1..R-1 (Ns = product of
@@ -302,37 +303,95 @@ __device__ __forceinline__ void fft_stages_ct(cplx<T>* lds, int nlines, int lstr
   }
 }
 
-// Butterflies per thread of the runtime-N engine: nb*nlines <= TILE_ELEMS/R
-// and TPL = floor(256/nlines) >= (256 - nlines)/nlines, so nb/TPL <=
-// (TILE_ELEMS/R)/(256 - MAXLINES).
-template <int R, int TILE_ELEMS, int MAXLINES> constexpr int fft_maxq_rt() {
-  return (TILE_ELEMS / R) / (FFT_THREADS - MAXLINES) + 1;
+// Runtime N: one wave per line, 64 butterflies a pass, so a line's stages need
+// no workgroup barrier (a wave's LDS accesses are carried out in order) and the
+// register arrays stay small for any N <= FFT_MAX_N.  (The threads of a
+// workgroup sharing all lines, as below for compile-time N, needs arrays sized
+// for the worst N, 190 to 256 registers.  Measured at N = 300, float: y pass
+// 0.37 -> 0.15 ms, assignment 0.66 -> 0.38, shell y pass of 20 shells 0.50 ->
+// 0.28, shell x pass 3.9 -> 1.02.  At compile-time N the shared form stays: with
+// 64 lanes a line 40 to 45 of them work at N = 360, and the y pass of 16 boxes
+// of 128 took 0.144 instead of 0.100 ms.)
+constexpr int FFT_MAX_N = 1024;
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int R, int S, typename T>
+__device__ __forceinline__ void fft_stage_wave(cplx<T>* base, int N, int Ns,
+                                               const cplx<T>* __restrict__ tw) {
+  constexpr int MAXQ = (FFT_MAX_N / R + 63) / 64;
+  const int nb = N / R, lane = (int)threadIdx.x & 63;
+  // j / Ns for j < 1024 by a multiplication (Ns > 1)
+  const unsigned magic = Ns > 1 ? 0xffffffffu / (unsigned)Ns + 1u : 0u;
+  cplx<T> v[MAXQ][R];
+  int kk[MAXQ];
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {
+    const int j = lane + q * 64;
+    kk[q] = 0;
+    if (j < nb) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[q][r] = base[j + r * nb];
+      const int k = Ns > 1 ? j - (int)__umulhi((unsigned)j, magic) * Ns : 0;
+      kk[q] = k;
+      // the first stage's row is ones: it is multiplied by it all the same, since
+      // which products the compiler fuses in dftR depends on where its inputs
+      // come from (the last bit of a float32 DFT of 9 otherwise differs)
+      const cplx<T>* w = tw + k * (R - 1);
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        cplx<T> wr = w[r - 1];
+        if (S > 0) wr.im = -wr.im;
+        v[q][r] = v[q][r] * wr;
+      }
+      dftR<R, S>(v[q]);
+    }
+  }
+  wave_lds_fence();
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {
+    const int j = lane + q * 64;
+    if (j < nb) {
+      const int k = kk[q];
+      cplx<T>* dst = base + (j - k) * R + k;
+#pragma unroll
+      for (int r = 0; r < R; ++r) dst[r * Ns] = v[q][r];
+    }
+  }
+  wave_lds_fence();
 }
 
 // Transform every line of the tile in place.  N > 0: compile-time length;
-// N == 0: runtime length sh.N with at most MAXLINES*sh.N <= TILE_ELEMS.
+// N == 0: runtime length sh.N.
 template <int N, int S, typename T, int MAXLINES, int TILE_ELEMS>
 __device__ __forceinline__ void fft_tile(cplx<T>* lds, const FftShape& sh, int nlines, int lstride,
                                          const cplx<T>* __restrict__ tw) {
   if constexpr (N > 0) {
     fft_stages_ct<N, 0, 1, 0, S, T, MAXLINES>(lds, nlines, lstride, tw);
   } else {
-    const int TPL = FFT_THREADS / (nlines > 0 ? nlines : 1);
-    int Ns = 1, off = 0;
-    for (int s = 0; s < sh.nstages; ++s) {
-      const int R = sh.radix[s];
-      const cplx<T>* t = tw + off;
-      switch (R) {
-        case 9: fft_stage<9, S, T, fft_maxq_rt<9, TILE_ELEMS, MAXLINES>()>(lds, sh.N, Ns, TPL, nlines, lstride, t); break;
-        case 8: fft_stage<8, S, T, fft_maxq_rt<8, TILE_ELEMS, MAXLINES>()>(lds, sh.N, Ns, TPL, nlines, lstride, t); break;
-        case 5: fft_stage<5, S, T, fft_maxq_rt<5, TILE_ELEMS, MAXLINES>()>(lds, sh.N, Ns, TPL, nlines, lstride, t); break;
-        case 4: fft_stage<4, S, T, fft_maxq_rt<4, TILE_ELEMS, MAXLINES>()>(lds, sh.N, Ns, TPL, nlines, lstride, t); break;
-        case 3: fft_stage<3, S, T, fft_maxq_rt<3, TILE_ELEMS, MAXLINES>()>(lds, sh.N, Ns, TPL, nlines, lstride, t); break;
-        default: fft_stage<2, S, T, fft_maxq_rt<2, TILE_ELEMS, MAXLINES>()>(lds, sh.N, Ns, TPL, nlines, lstride, t); break;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (int line = wave; line < nlines; line += FFT_THREADS / 64) {
+      cplx<T>* base = lds + line * lstride;
+      int Ns = 1, off = 0;
+      for (int s = 0; s < sh.nstages; ++s) {
+        const int R = sh.radix[s];
+        const cplx<T>* t = tw + off;
+        switch (R) {
+          case 9: fft_stage_wave<9, S, T>(base, sh.N, Ns, t); break;
+          case 8: fft_stage_wave<8, S, T>(base, sh.N, Ns, t); break;
+          case 5: fft_stage_wave<5, S, T>(base, sh.N, Ns, t); break;
+          case 4: fft_stage_wave<4, S, T>(base, sh.N, Ns, t); break;
+          case 3: fft_stage_wave<3, S, T>(base, sh.N, Ns, t); break;
+          default: fft_stage_wave<2, S, T>(base, sh.N, Ns, t); break;
+        }
+        off += Ns * (R - 1);
+        Ns *= R;
       }
-      off += Ns * (R - 1);
-      Ns *= R;
     }
+    __syncthreads();
   }
 }
 
