@@ -225,10 +225,35 @@ __device__ __forceinline__ int wrap1(int c, int N) {
   return c < 0 ? c + N : (c >= N ? c - N : c);
 }
 
-// LDS: int64 accumulators acc[line][x][grid] (16 B per cell); with FFTX the
-// same memory then holds the complex lines (row stride N+1) and the twiddles.
-// Box blockIdx.y of a batch: its sorted records (from bs.poff), tile
-// offsets [box][ntiles + 1] and grid out [box][N^3].
+// The rows of work of a tile: entries (record, grid, z stencil row).  A tile
+// has at most ASSIGN_TZ z rows, so a particle gives at most that many per grid;
+// after each batch of FFT_THREADS particles at most FFT_THREADS - 1 entries stay.
+constexpr int ASSIGN_TZ = ASSIGN_LINES / PSX_ASSIGN_TY < 4 ? ASSIGN_LINES / PSX_ASSIGN_TY : 4;
+constexpr int ASSIGN_QUEUE = FFT_THREADS * (2 * ASSIGN_TZ + 1);
+constexpr size_t ASSIGN_QUEUE_BYTES = ASSIGN_QUEUE * (sizeof(unsigned) + 1);
+
+// LDS: int64 accumulators acc[line][x][grid] (16 B per cell) and the queue of
+// entries; with FFTX the same memory then holds the complex lines (row stride
+// N+1) and the twiddles.  Box blockIdx.y of a batch: its sorted records (from
+// bs.poff), tile offsets [box][ntiles + 1] and grid out [box][N^3].
+//
+// A tile's workgroup visits the particles of twelve tiles, and of the 32
+// stencil rows of a particle about one in twelve is its own: with a thread a
+// particle most lanes idle behind masks.  So the workgroup first lists, 256
+// particles at a time, the (particle, grid, z row) entries that land in the
+// tile, and then works through full rounds of 256 entries, each thread
+// recomputing its particle's stencil and adding up to four y rows.  Integer
+// sums, so neither the order of the list nor that of the atomics matters.
+//
+// The other half of the kernel is the lines: zeroing, conversion, FFT and
+// store.  A thread converts and stores cells of one line, with no index
+// division, all of them between two barriers.  Measured, float, before and
+// after both changes: N = 360 with 2e4 points 0.41 -> 0.30 ms, 1e6 0.563 ->
+// 0.478, 4e6 1.19 -> 1.09; N = 512, 4e6 2.16 -> 1.96; N = 256, 3e5 0.174 ->
+// 0.151; double, N = 360, 1e6 0.655 -> 0.553; a 40^3 grid with 320 points a line
+// (200 workgroups, fewer than CUs) 0.339 -> 0.354.  (Fixed point by adding 1.5
+// * 2^52 instead of the float64 conversion, under a branch on the weight's
+// size: 0.51 -> 0.57 at N = 360.)
 template <typename T, int NC, bool FFTX>
 __global__ __launch_bounds__(FFT_THREADS) void k_assign_lines(
     const float4* __restrict__ rec, const unsigned* __restrict__ tile_off, const AssignBoxes bs,
@@ -243,15 +268,18 @@ __global__ __launch_bounds__(FFT_THREADS) void k_assign_lines(
   extern __shared__ __align__(16) unsigned char smem_raw[];
   unsigned long long* acc = reinterpret_cast<unsigned long long*>(smem_raw);
   __shared__ int src[64];
-  __shared__ int64_t sbeg[64];
+  __shared__ unsigned sbeg[64];
   __shared__ int64_t pre[65];
-  __shared__ int nsrc_s;
+  __shared__ int nsrc_s, nq_s;
   const int N = n_of<NC>(sh);
   const int y0 = (int)(blockIdx.x % at.nty) * at.ty, z0 = (int)(blockIdx.x / at.nty) * at.tz;
   const int y1 = min(y0 + at.ty, N), z1 = min(z0 + at.tz, N);
   const int nl = at.ty * at.tz;
   const int ncell = nl * N;
-  for (int i = threadIdx.x; i < 2 * ncell; i += FFT_THREADS) acc[i] = 0ull;
+  unsigned* q_rec = reinterpret_cast<unsigned*>(smem_raw + (size_t)16 * ncell);
+  unsigned char* q_row = reinterpret_cast<unsigned char*>(q_rec + ASSIGN_QUEUE);
+  for (int i = threadIdx.x; i < ncell; i += FFT_THREADS)
+    reinterpret_cast<ulonglong2*>(acc)[i] = make_ulonglong2(0ull, 0ull);
   if (threadIdx.x == 0) {
     int sy[8], sz[8];
     const int ny = source_tiles(y0, y1, N, at.ty, sy);
@@ -260,127 +288,185 @@ __global__ __launch_bounds__(FFT_THREADS) void k_assign_lines(
     for (int b = 0; b < nz; ++b)
       for (int a = 0; a < ny; ++a) src[n++] = sz[b] * at.nty + sy[a];
     nsrc_s = n;
+    nq_s = 0;
   }
   __syncthreads();
   const int nsrc = nsrc_s;
   if ((int)threadIdx.x < nsrc) {
     const unsigned key = (unsigned)src[threadIdx.x];
     // records of tile key: [tile_off[key], tile_off[key + 1])
-    sbeg[threadIdx.x] = np > 0 ? (int64_t)tile_off[key] : 0;
-    pre[threadIdx.x + 1] = np > 0 ? (int64_t)tile_off[key + 1] : 0;  // range end for now
+    const unsigned beg = np > 0 ? tile_off[key] : 0u;
+    sbeg[threadIdx.x] = beg;
+    pre[threadIdx.x + 1] = np > 0 ? (int64_t)(tile_off[key + 1] - beg) : 0;  // length for now
   }
   __syncthreads();
   if (threadIdx.x == 0) {
     int64_t s = 0;
     pre[0] = 0;
     for (int u = 0; u < nsrc; ++u) {
-      s += pre[u + 1] - sbeg[u];
+      s += pre[u + 1];
       pre[u + 1] = s;
     }
   }
   __syncthreads();
   const int64_t total = pre[nsrc];
-  int s = 0;
-  constexpr int U = 4;  // particle records loaded ahead of their use
-  for (int64_t q0 = threadIdx.x; q0 < total; q0 += FFT_THREADS * U) {
-    float4 rq[U];
+  const int lane = (int)(threadIdx.x & 63);
+  const unsigned long long below = (1ull << lane) - 1ull;
+  auto add_row = [&](const float4& r, int code) {
+    const bool shift = (code & 4) != 0;
+    const int g = shift ? 1 : 0, c = code & 3;
+    int ex, ey, ez;
+    T wx[4], wy[4], wz[4];
+    pcs_weights(pcs_coord(r.x, pm, shift, N, &ex), wx);
+    pcs_weights(pcs_coord(r.y, pm, shift, N, &ey), wy);
+    pcs_weights(pcs_coord(r.z, pm, shift, N, &ez), wz);
+    const T wzc = c & 2 ? (c & 1 ? wz[3] : wz[2]) : (c & 1 ? wz[1] : wz[0]);
+    const int zrow = (wrap1(ez + c - 1, N) - z0) * at.ty;
+    const T we = (T)r.w;
+    int ix[4];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t q = q0 + (int64_t)u * FFT_THREADS;
-      if (q < total) {
-        while (q >= pre[s + 1]) ++s;
-        rq[u] = rec[sbeg[s] + (q - pre[s])];
+    for (int a = 0; a < 4; ++a) ix[a] = 2 * wrap1(ex + a - 1, N) + g;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int yy = wrap1(ey + b - 1, N);
+      if (yy < y0 || yy >= y1) continue;
+      unsigned long long* row = acc + 2 * (zrow + yy - y0) * N;
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        // estimator.f:380-508: hx*hy*hz*we, left to right
+        const T v = wmul(wmul(wmul(wx[a], wy[b]), wzc), we);
+        const long long qv = __double2ll_rn((double)v * scale);
+        atomicAdd(row + ix[a], (unsigned long long)qv);
       }
     }
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    if (q0 + (int64_t)u * FFT_THREADS >= total) break;
-    const float4 r = rq[u];
-    const float p[3] = {r.x, r.y, r.z};
-    const T we = (T)r.w;
+  };
+  int s = 0;
+  unsigned at_rec = 0;  // this thread's record of the batch
+  auto locate = [&](int64_t q) {
+    while (q >= pre[s + 1]) ++s;
+    return sbeg[s] + (unsigned)(q - pre[s]);
+  };
+  float4 nxt = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if ((int64_t)threadIdx.x < total) nxt = rec[at_rec = locate(threadIdx.x)];
+  for (int64_t q0 = 0; q0 < total; q0 += FFT_THREADS) {
+    const float4 r = nxt;
+    const unsigned my_rec = at_rec;
+    const bool has = q0 + threadIdx.x < total;
+    if (q0 + FFT_THREADS + threadIdx.x < total) nxt = rec[at_rec = locate(q0 + FFT_THREADS + threadIdx.x)];
+    // which of the 2 x 4 z stencil rows land in the tile
+    unsigned hits = 0;
 #pragma unroll
     for (int g = 0; g < 2; ++g) {
       int cy, cz;
-      const float hy = pcs_coord(p[1], pm, g == 1, N, &cy);
-      const float hz = pcs_coord(p[2], pm, g == 1, N, &cz);
-      int ly[4], lz[4];
-      unsigned my = 0, mz = 0;
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const int yy = wrap1(cy + a - 1, N), zz = wrap1(cz + a - 1, N);
-        ly[a] = yy - y0;
-        lz[a] = zz - z0;
-        if (yy >= y0 && yy < y1) my |= 1u << a;
-        if (zz >= z0 && zz < z1) mz |= 1u << a;
-      }
-      if (my == 0 || mz == 0) continue;
-      int cx;
-      T wx[4], wy[4], wz[4];
-      pcs_weights(pcs_coord(p[0], pm, g == 1, N, &cx), wx);
-      pcs_weights(hy, wy);
-      pcs_weights(hz, wz);
-      int ix[4];
-#pragma unroll
-      for (int a = 0; a < 4; ++a) ix[a] = wrap1(cx + a - 1, N);
+      (void)pcs_coord(r.y, pm, g == 1, N, &cy);
+      (void)pcs_coord(r.z, pm, g == 1, N, &cz);
+      bool hit_y = false;
+      unsigned hz = 0;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        if (!((mz >> c) & 1u)) continue;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          if (!((my >> b) & 1u)) continue;
-          const int row = (lz[c] * at.ty + ly[b]) * N;
-#pragma unroll
-          for (int a = 0; a < 4; ++a) {
-            // estimator.f:380-508: hx*hy*hz*we, left to right
-            const T v = wmul(wmul(wmul(wx[a], wy[b]), wz[c]), we);
-            const long long qv = __double2ll_rn((double)v * scale);
-            atomicAdd(acc + 2 * (row + ix[a]) + g, (unsigned long long)qv);
-          }
-        }
+        const int yy = wrap1(cy + c - 1, N), zz = wrap1(cz + c - 1, N);
+        hit_y = hit_y || (yy >= y0 && yy < y1);
+        if (zz >= z0 && zz < z1) hz |= 1u << (4 * g + c);
       }
+      if (has && hit_y) hits |= hz;
     }
-  }
+    // the wave's entries at `base`, stencil row by stencil row
+    int n_wave = 0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) n_wave += __popcll(__ballot((hits >> k) & 1u));
+    int base = 0;
+    if (lane == 0 && n_wave > 0) base = atomicAdd(&nq_s, n_wave);
+    base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const unsigned long long m = __ballot((hits >> k) & 1u);
+      if ((hits >> k) & 1u) {
+        const int i = base + __popcll(m & below);
+        q_rec[i] = my_rec;
+        q_row[i] = (unsigned char)k;
+      }
+      base += __popcll(m);
+    }
+    __syncthreads();
+    const int n = nq_s;
+    const int work = q0 + FFT_THREADS < total ? n / FFT_THREADS * FFT_THREADS : n;
+    // two rounds at a time, so that their records are loaded together
+    for (int i0 = (int)threadIdx.x; i0 < work; i0 += 2 * FFT_THREADS) {
+      const int i1 = i0 + FFT_THREADS;
+      const float4 r0 = rec[q_rec[i0]];
+      float4 r1 = r0;
+      if (i1 < work) r1 = rec[q_rec[i1]];
+      add_row(r0, q_row[i0]);
+      if (i1 < work) add_row(r1, q_row[i1]);
+    }
+    // the rest (fewer than FFT_THREADS) to the front
+    unsigned kr = 0;
+    unsigned char kc = 0;
+    const bool keep = work + (int)threadIdx.x < n;
+    if (keep) { kr = q_rec[work + threadIdx.x]; kc = q_row[work + threadIdx.x]; }
+    __syncthreads();
+    if (keep) { q_rec[threadIdx.x] = kr; q_row[threadIdx.x] = kc; }
+    if (threadIdx.x == 0) nq_s = n - work;
+    __syncthreads();
   }
   __syncthreads();
+  // a thread converts and stores the cells x = x0, x0 + TP, ... of one line
   const double inv = 1.0 / scale;
+  const int TP = FFT_THREADS / nl;
+  const int line = (int)threadIdx.x / TP, xf = (int)threadIdx.x - line * TP;
+  const int ly = line % at.ty, lz = line / at.ty;
+  const bool stored = line < nl && y0 + ly < y1 && z0 + lz < z1;
+  cplx<T>* dst = out + ((int64_t)(z0 + lz) * N + (y0 + ly)) * N;
   if constexpr (!FFTX) {
-    for (int e = threadIdx.x; e < ncell; e += FFT_THREADS) {
-      const int line = e / N, x = e - line * N;
-      const int y = y0 + line % at.ty, z = z0 + line / at.ty;
-      if (y < y1 && z < z1)
-        out[((int64_t)z * N + y) * N + x] = mk((T)((double)(long long)acc[2 * e] * inv),
-                                               (T)((double)(long long)acc[2 * e + 1] * inv));
-    }
+    if (stored)
+      for (int x = xf; x < N; x += TP) {
+        const unsigned long long* a = acc + 2 * (line * N + x);
+        dst[x] = mk((T)((double)(long long)a[0] * inv), (T)((double)(long long)a[1] * inv));
+      }
   } else {
-    // Convert in place to complex lines of stride N+1.  Cell e moves from
-    // byte 16e to byte sizeof(cplx<T>)*(e + line): for 8-byte complex the
-    // destination lies in cells already read when rounds go up, for 16-byte
-    // complex in cells already read when rounds go down.
+    // To complex lines of stride N+1 in the same memory.  Compile-time N: all
+    // of a thread's cells are in registers between two barriers.  Runtime N:
+    // CR rounds of cells at a time; cell e moves from byte 16e to byte
+    // sizeof(cplx<T>)*(e + line), for 8-byte complex into cells already read
+    // when the batches go up, for 16-byte complex when they go down.
     cplx<T>* lds = reinterpret_cast<cplx<T>*>(smem_raw);
     const int lstride = N + 1;
-    const int nround = (ncell + FFT_THREADS - 1) / FFT_THREADS;
-    for (int r = 0; r < nround; ++r) {
-      const int rr = sizeof(cplx<T>) < 16 ? r : nround - 1 - r;
-      const int e = rr * FFT_THREADS + threadIdx.x;
-      cplx<T> v = mk(T(0), T(0));
-      if (e < ncell)
-        v = mk((T)((double)(long long)acc[2 * e] * inv), (T)((double)(long long)acc[2 * e + 1] * inv));
+    auto cell = [&](int e) {
+      return mk((T)((double)(long long)acc[2 * e] * inv), (T)((double)(long long)acc[2 * e + 1] * inv));
+    };
+    if constexpr (NC > 0) {
+      constexpr int TPC = FFT_THREADS / assign_lines_max<T, NC>(), U = (NC + TPC - 1) / TPC;
+      cplx<T> v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        v[u] = cell(min(line, nl - 1) * N + min(xf + u * TP, N - 1));
       __syncthreads();
-      if (e < ncell) {
-        const int line = e / N;
-        lds[e + line] = v;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (line < nl && xf + u * TP < N) lds[line * lstride + xf + u * TP] = v[u];
+    } else {
+      constexpr int CR = 8, CB = CR * FFT_THREADS;
+      const int nbatch = (ncell + CB - 1) / CB;
+      for (int bt = 0; bt < nbatch; ++bt) {
+        const int e0 = (sizeof(cplx<T>) < 16 ? bt : nbatch - 1 - bt) * CB + (int)threadIdx.x;
+        cplx<T> v[CR];
+#pragma unroll
+        for (int u = 0; u < CR; ++u) v[u] = cell(min(e0 + u * FFT_THREADS, ncell - 1));
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < CR; ++u) {
+          const int e = e0 + u * FFT_THREADS;
+          if (e < ncell) lds[e + e / N] = v[u];
+        }
+        __syncthreads();
       }
-      __syncthreads();
     }
     cplx<T>* twl = lds + nl * lstride;
     stage_twiddles(twl, tw, N);
     __syncthreads();
     fft_tile<NC, 1, T, assign_lines_max<T, NC>(), TileCfg<T>::ELEMS>(lds, sh, nl, lstride, twl);
-    for (int e = threadIdx.x; e < ncell; e += FFT_THREADS) {
-      const int line = e / N, x = e - line * N;
-      const int y = y0 + line % at.ty, z = z0 + line / at.ty;
-      if (y < y1 && z < z1) out[((int64_t)z * N + y) * N + x] = lds[line * lstride + x];
-    }
+    if (stored)
+      for (int x = xf; x < N; x += TP) dst[x] = lds[line * lstride + x];
   }
 }
 
@@ -401,7 +487,7 @@ static int assign_lines_n(psx_ctx* ctx, const float4* rec, const unsigned* off,
   const FftPlan* p;
   PSX_TRY(get_fft_plan(ctx, N, &p));
   const size_t nl = (size_t)at.ty * at.tz;
-  const size_t acc_bytes = 16 * nl * N;
+  const size_t acc_bytes = 16 * nl * N + ASSIGN_QUEUE_BYTES;
   const dim3 blocks((unsigned)(at.nty * at.ntz), (unsigned)nbox);
   if (fft_x) {
     const size_t fft_bytes = sizeof(cplx<T>) * (nl * (N + 1) + N);
