@@ -227,10 +227,9 @@ __device__ __forceinline__ int wrap1(int c, int N) {
 
 // The rows of work of a tile: entries (record, grid, z stencil row).  A tile
 // has at most ASSIGN_TZ z rows, so a particle gives at most that many per grid;
-// after each batch of FFT_THREADS particles at most FFT_THREADS - 1 entries stay.
+// after a batch (one particle a thread) fewer entries than threads stay.
 constexpr int ASSIGN_TZ = ASSIGN_LINES / PSX_ASSIGN_TY < 4 ? ASSIGN_LINES / PSX_ASSIGN_TY : 4;
-constexpr int ASSIGN_QUEUE = FFT_THREADS * (2 * ASSIGN_TZ + 1);
-constexpr size_t ASSIGN_QUEUE_BYTES = ASSIGN_QUEUE * (sizeof(unsigned) + 1);
+__host__ __device__ constexpr int assign_queue(int threads) { return threads * (2 * ASSIGN_TZ + 1); }
 
 // LDS: int64 accumulators acc[line][x][grid] (16 B per cell) and the queue of
 // entries; with FFTX the same memory then holds the complex lines (row stride
@@ -239,23 +238,23 @@ constexpr size_t ASSIGN_QUEUE_BYTES = ASSIGN_QUEUE * (sizeof(unsigned) + 1);
 //
 // A tile's workgroup visits the particles of twelve tiles, and of the 32
 // stencil rows of a particle about one in twelve is its own: with a thread a
-// particle most lanes idle behind masks.  So the workgroup first lists, 256
+// particle most lanes idle behind masks.  So the workgroup first lists, TH
 // particles at a time, the (particle, grid, z row) entries that land in the
-// tile, and then works through full rounds of 256 entries, each thread
+// tile, and then works through full rounds of TH entries, each thread
 // recomputing its particle's stencil and adding up to four y rows.  Integer
 // sums, so neither the order of the list nor that of the atomics matters.
+// The lines' part runs on FFT_THREADS threads, whatever TH.
 //
 // The other half of the kernel is the lines: zeroing, conversion, FFT and
 // store.  A thread converts and stores cells of one line, with no index
 // division, all of them between two barriers.  Measured, float, before and
 // after both changes: N = 360 with 2e4 points 0.41 -> 0.30 ms, 1e6 0.563 ->
 // 0.478, 4e6 1.19 -> 1.09; N = 512, 4e6 2.16 -> 1.96; N = 256, 3e5 0.174 ->
-// 0.151; double, N = 360, 1e6 0.655 -> 0.553; a 40^3 grid with 320 points a line
-// (200 workgroups, fewer than CUs) 0.339 -> 0.354.  (Fixed point by adding 1.5
-// * 2^52 instead of the float64 conversion, under a branch on the weight's
-// size: 0.51 -> 0.57 at N = 360.)
-template <typename T, int NC, bool FFTX>
-__global__ __launch_bounds__(FFT_THREADS) void k_assign_lines(
+// 0.151; double, N = 360, 1e6 0.655 -> 0.553.  (Fixed point by adding 1.5 * 2^52
+// instead of the float64 conversion, under a branch on the weight's size: 0.51
+// -> 0.57 at N = 360.)
+template <typename T, int NC, bool FFTX, int TH>
+__global__ __launch_bounds__(TH) void k_assign_lines(
     const float4* __restrict__ rec, const unsigned* __restrict__ tile_off, const AssignBoxes bs,
     FftShape sh, AssignTiling at, const cplx<T>* __restrict__ tw, cplx<T>* __restrict__ out) {
   const int box = blockIdx.y;
@@ -277,8 +276,8 @@ __global__ __launch_bounds__(FFT_THREADS) void k_assign_lines(
   const int nl = at.ty * at.tz;
   const int ncell = nl * N;
   unsigned* q_rec = reinterpret_cast<unsigned*>(smem_raw + (size_t)16 * ncell);
-  unsigned char* q_row = reinterpret_cast<unsigned char*>(q_rec + ASSIGN_QUEUE);
-  for (int i = threadIdx.x; i < ncell; i += FFT_THREADS)
+  unsigned char* q_row = reinterpret_cast<unsigned char*>(q_rec + assign_queue(TH));
+  for (int i = threadIdx.x; i < ncell; i += TH)
     reinterpret_cast<ulonglong2*>(acc)[i] = make_ulonglong2(0ull, 0ull);
   if (threadIdx.x == 0) {
     int sy[8], sz[8];
@@ -348,11 +347,11 @@ __global__ __launch_bounds__(FFT_THREADS) void k_assign_lines(
   };
   float4 nxt = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   if ((int64_t)threadIdx.x < total) nxt = rec[at_rec = locate(threadIdx.x)];
-  for (int64_t q0 = 0; q0 < total; q0 += FFT_THREADS) {
+  for (int64_t q0 = 0; q0 < total; q0 += TH) {
     const float4 r = nxt;
     const unsigned my_rec = at_rec;
     const bool has = q0 + threadIdx.x < total;
-    if (q0 + FFT_THREADS + threadIdx.x < total) nxt = rec[at_rec = locate(q0 + FFT_THREADS + threadIdx.x)];
+    if (q0 + TH + threadIdx.x < total) nxt = rec[at_rec = locate(q0 + TH + threadIdx.x)];
     // which of the 2 x 4 z stencil rows land in the tile
     unsigned hits = 0;
 #pragma unroll
@@ -389,17 +388,17 @@ __global__ __launch_bounds__(FFT_THREADS) void k_assign_lines(
     }
     __syncthreads();
     const int n = nq_s;
-    const int work = q0 + FFT_THREADS < total ? n / FFT_THREADS * FFT_THREADS : n;
+    const int work = q0 + TH < total ? n / TH * TH : n;
     // two rounds at a time, so that their records are loaded together
-    for (int i0 = (int)threadIdx.x; i0 < work; i0 += 2 * FFT_THREADS) {
-      const int i1 = i0 + FFT_THREADS;
+    for (int i0 = (int)threadIdx.x; i0 < work; i0 += 2 * TH) {
+      const int i1 = i0 + TH;
       const float4 r0 = rec[q_rec[i0]];
       float4 r1 = r0;
       if (i1 < work) r1 = rec[q_rec[i1]];
       add_row(r0, q_row[i0]);
       if (i1 < work) add_row(r1, q_row[i1]);
     }
-    // the rest (fewer than FFT_THREADS) to the front
+    // the rest (fewer than TH) to the front
     unsigned kr = 0;
     unsigned char kc = 0;
     const bool keep = work + (int)threadIdx.x < n;
@@ -410,6 +409,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_assign_lines(
     __syncthreads();
   }
   __syncthreads();
+  if (TH > FFT_THREADS && threadIdx.x >= FFT_THREADS) return;  // whole waves: barriers go on without them
   // a thread converts and stores the cells x = x0, x0 + TP, ... of one line
   const double inv = 1.0 / scale;
   const int TP = FFT_THREADS / nl;
@@ -480,30 +480,42 @@ int fixed_point_exponent(double wsum_abs) {
   return e;
 }
 
+template <typename T, int NC, bool FFTX, int TH>
+static int assign_lines_th(psx_ctx* ctx, const float4* rec, const unsigned* off,
+                           const AssignBoxes& bs, int nbox, int N, AssignTiling at, cplx<T>* grid) {
+  const FftPlan* p;
+  PSX_TRY(get_fft_plan(ctx, N, &p));
+  const size_t nl = (size_t)at.ty * at.tz;
+  size_t lds = 16 * nl * N + assign_queue(TH) * (sizeof(unsigned) + 1);
+  if (FFTX) lds = std::max(lds, sizeof(cplx<T>) * (nl * (N + 1) + N));
+  auto kern = k_assign_lines<T, NC, FFTX, TH>;
+  PSX_TRY(set_lds(kern, lds));
+  launch_timed(ctx, "k_assign_lines", kern, dim3((unsigned)(at.nty * at.ntz), (unsigned)nbox),
+               dim3(TH), lds, rec, off, bs, p->shape, at, plan_tw<T>(p), grid);
+  PSX_CHECK_LAUNCH();
+  return PSX_OK;
+}
+
+// Small grids have fewer workgroups than the chip takes at once, and a wave of
+// one waits for its LDS atomics and records: up to two workgroups a CU (512
+// tiles, N = 64) they get 16 waves instead of 4.  Measured, float, 256 against
+// 1024 threads: N = 40 with 2e4 points 0.030 -> 0.021 ms, 512000 0.358 -> 0.184;
+// N = 64, 2e4 0.018 -> 0.017, 2e6 0.60 -> 0.415; above, the wide ones lose what
+// is sparse: N = 80 (800 tiles) 2e4 0.026 -> 0.046, 5e5 0.168 -> 0.189, N = 128
+// 2e4 0.034 -> 0.056.
+constexpr int ASSIGN_WIDE_TILES = 512, ASSIGN_WIDE_THREADS = 1024;
+
 template <typename T, int NC>
 static int assign_lines_n(psx_ctx* ctx, const float4* rec, const unsigned* off,
                           const AssignBoxes& bs, int nbox, int N, AssignTiling at, cplx<T>* grid,
                           bool fft_x) {
-  const FftPlan* p;
-  PSX_TRY(get_fft_plan(ctx, N, &p));
-  const size_t nl = (size_t)at.ty * at.tz;
-  const size_t acc_bytes = 16 * nl * N + ASSIGN_QUEUE_BYTES;
-  const dim3 blocks((unsigned)(at.nty * at.ntz), (unsigned)nbox);
-  if (fft_x) {
-    const size_t fft_bytes = sizeof(cplx<T>) * (nl * (N + 1) + N);
-    const size_t lds = acc_bytes > fft_bytes ? acc_bytes : fft_bytes;
-    auto kern = k_assign_lines<T, NC, true>;
-    PSX_TRY(set_lds(kern, lds));
-    launch_timed(ctx, "k_assign_lines", kern, blocks, dim3(FFT_THREADS), lds, rec, off, bs,
-                 p->shape, at, plan_tw<T>(p), grid);
-  } else {
-    auto kern = k_assign_lines<T, 0, false>;
-    PSX_TRY(set_lds(kern, acc_bytes));
-    launch_timed(ctx, "k_assign_lines", kern, blocks, dim3(FFT_THREADS), acc_bytes, rec, off, bs,
-                 p->shape, at, plan_tw<T>(p), grid);
+  if (!fft_x)
+    return assign_lines_th<T, 0, false, FFT_THREADS>(ctx, rec, off, bs, nbox, N, at, grid);
+  if constexpr (NC <= 64) {
+    if ((int64_t)at.nty * at.ntz * nbox <= ASSIGN_WIDE_TILES)
+      return assign_lines_th<T, NC, true, ASSIGN_WIDE_THREADS>(ctx, rec, off, bs, nbox, N, at, grid);
   }
-  PSX_CHECK_LAUNCH();
-  return PSX_OK;
+  return assign_lines_th<T, NC, true, FFT_THREADS>(ctx, rec, off, bs, nbox, N, at, grid);
 }
 
 #define PSX_CASE_N(n)                                                                         \

@@ -44,3 +44,33 @@ def test_assignment_list_edges(N, n, tile, prec):
     tol = 1e-11 if prec == "fp64" else 5e-7
     for got, ref in ((out.real, A), (out.imag, B)):
         assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("N,n,tile", [(4, 1025, False), (32, 1, False), (40, 1023, True),
+                                      (40, 30000, True), (64, 5000, False), (72, 5000, False)])
+def test_small_grids_match_stages(N, n, tile, prec):
+    """The assignment with the x pass, in wide workgroups up to N = 64, against
+    psx_assign_quad and psx_fft3d on every element (float32 FFT rounding 2e-6,
+    float64 1e-12 of the largest)."""
+    print("[case] small grid", N, n, tile, prec, flush=True)
+    Lbox = 100.0
+    rng = np.random.default_rng(N + n)
+    xyz = rng.uniform(0, Lbox, size=(3, n))
+    if tile:
+        xyz[1:] *= 2.0 / N
+    x = torch.from_numpy(xyz.astype(np.float32)).to(DEV)
+    cd = torch.complex128 if prec == "fp64" else torch.complex64
+    p = L.PREC[prec]
+    ctx = L.Context(0)
+    got = torch.empty((N, N, N // 2 + 1), dtype=cd, device=DEV)
+    ctx.call("psx_fft_periodic", L.ptr(x), None, n, N, Lbox, float(n), float(n), L.ptr(got), p)
+    grid = torch.empty((N, N, N), dtype=cd, device=DEV)
+    ref = torch.empty_like(got)
+    ctx.call("psx_assign_quad", L.ptr(x), None, n, N, float(np.float32(N / Lbox)), 0.0, 0.0,
+             float(np.float32(Lbox * (1 - 1e-6))), float(n), L.ptr(grid), p)
+    ctx.call("psx_fft3d", L.ptr(grid), N, 1, p)
+    ctx.call("psx_fcomb_periodic", L.ptr(grid), L.ptr(ref), N, float(n), p)
+    tol = (1e-12 if prec == "fp64" else 2e-6) * float(ref.abs().max())
+    assert float((got - ref).abs().max()) <= tol
+    ctx.close()
