@@ -33,10 +33,10 @@ def run_batch(ctx, xyzs, ws, Lboxes, Ngrid, step, Ncut, Nmax, precision, device,
     boxes = (L.PsxBox * nbox)()
     keep = []
     sums = []
-    for b in range(nbox):
-        x = P._positions(xyzs[b], device)
+    xs = [P._positions(x, device) for x in xyzs]
+    wds = P._weights_list([None] * nbox if ws is None else ws, [x.shape[1] for x in xs], device)
+    for b, (x, (wd, sw, sabs)) in enumerate(zip(xs, wds)):
         n = x.shape[1]
-        wd, sw, sabs = P._weights(None if ws is None else ws[b], n, device)
         keep += [x, wd]
         Lb = float(Lboxes[b])
         kf = 2 * np.pi / Lb
@@ -73,9 +73,10 @@ def Bk_periodic_batch(xyzs, ws=None, Lbox=2600., Ngrid=360, step=3, Ncut=3, Nmax
         out7, _, _, sums, ijl, tc, _ = run_batch(ctx, xyzs[sl], None if ws is None else ws[sl],
                                                  Lboxes[sl], Ngrid, step, Ncut, Nmax, precision,
                                                  device)
+        sides = P._sides(ijl, step, tc > 0)
         fin = out7.cpu().numpy()
         for b, (n, sw, nbar, kf) in enumerate(sums):
-            bispec = P._assemble(ijl, step, fin[b][:, :len(ijl)], tc > 0)
+            bispec = P._assemble({k: v.copy() for k, v in sides.items()}, fin[b][:, :len(ijl)])
             d = {k: bispec[k] for k in ('i_k1', 'i_k2', 'i_k3', 'p0k1', 'p0k2', 'p0k3', 'b123',
                                         'q123', 'counts')}
             d['meta'] = {'Lbox': Lboxes[s + b], 'Ngrid': Ngrid, 'step': step, 'Ncut': Ncut,

@@ -52,7 +52,7 @@ def _half_arg(a, Ngrid, device):
     t = torch.from_numpy(np.ascontiguousarray(arr.transpose(2, 1, 0))).to(torch.device("cuda", device))
 
     def back():
-        arr[...] = t.cpu().numpy().transpose(2, 1, 0)
+        arr[...] = L.to_numpy(t).transpose(2, 1, 0)
     return t, prec, back
 
 
