@@ -290,16 +290,63 @@ __device__ __forceinline__ void fft_stage(cplx<T>* lds, IntN N, IntNs Ns, IntTPL
 
 // Compile-time N: stages unrolled by recursion over the radix sequence; TW
 // is the offset of the stage's twiddle rows in the table.
-template <int N, int STAGE, int NS, int TW, int S, typename T, int MAXLINES>
+template <int N, int STAGE, int NS, int TW, int S, typename T, int MAXLINES, int LAST>
 __device__ __forceinline__ void fft_stages_ct(cplx<T>* lds, int nlines, int lstride,
                                               const cplx<T>* __restrict__ tw) {
   constexpr FftShape sh = fft_shape_of(N);
-  if constexpr (STAGE < sh.nstages) {
+  if constexpr (STAGE < LAST) {
     constexpr int R = sh.radix[STAGE];
     constexpr int TPL = FFT_THREADS / MAXLINES;
     constexpr int MAXQ = (N / R + TPL - 1) / TPL;
     fft_stage<R, S, T, MAXQ>(lds, IntC<N>(), IntC<NS>(), IntC<TPL>(), nlines, lstride, tw + TW);
-    fft_stages_ct<N, STAGE + 1, NS * R, TW + NS * (R - 1), S, T, MAXLINES>(lds, nlines, lstride, tw);
+    fft_stages_ct<N, STAGE + 1, NS * R, TW + NS * (R - 1), S, T, MAXLINES, LAST>(lds, nlines,
+                                                                                lstride, tw);
+  }
+}
+
+// The lines of the tile transformed, the last stage's butterflies not back to
+// LDS but to store(line, n, value): n = j + r N/R, so that a line's lanes hold
+// consecutive n (compile-time N).
+template <int N, int S, typename T, int MAXLINES, typename Store>
+__device__ __forceinline__ void fft_tile_store(cplx<T>* lds, int nlines, int lstride,
+                                               const cplx<T>* __restrict__ tw, Store store) {
+  constexpr FftShape sh = fft_shape_of(N);
+  static_assert(sh.nstages > 1, "one stage");
+  constexpr int LAST = sh.nstages - 1, R = sh.radix[LAST], NB = N / R;
+  constexpr int TPL = FFT_THREADS / MAXLINES, MAXQ = (NB + TPL - 1) / TPL;
+  fft_stages_ct<N, 0, 1, 0, S, T, MAXLINES, LAST>(lds, nlines, lstride, tw);
+  // the earlier stages have NB - 1 twiddles (the sum of Ns (R - 1) telescopes)
+  const cplx<T>* tl = tw + NB - 1;
+  const int line = (int)threadIdx.x / TPL, lane = (int)threadIdx.x - line * TPL;
+  const bool act = line < nlines;
+  const cplx<T>* base = lds + line * lstride;
+  cplx<T> v[MAXQ][R];
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {
+    const int j = lane + q * TPL;
+    if (act && j < NB) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[q][r] = base[j + r * NB];
+      const cplx<T>* w = tl + j * (R - 1);
+#pragma unroll
+      for (int r = 1; r < R; ++r) {
+        cplx<T> wr = w[r - 1];
+        if (S > 0) wr.im = -wr.im;
+        v[q][r] = v[q][r] * wr;
+      }
+      dftR<R, S>(v[q]);
+    }
+  }
+  // between the two loops as in fft_stage: which products the compiler fuses
+  // in dftR would otherwise depend on the stores
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int q = 0; q < MAXQ; ++q) {
+    const int j = lane + q * TPL;
+    if (act && j < NB) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) store(line, j + r * NB, v[q][r]);
+    }
   }
 }
 
@@ -370,7 +417,7 @@ template <int N, int S, typename T, int MAXLINES, int TILE_ELEMS>
 __device__ __forceinline__ void fft_tile(cplx<T>* lds, const FftShape& sh, int nlines, int lstride,
                                          const cplx<T>* __restrict__ tw) {
   if constexpr (N > 0) {
-    fft_stages_ct<N, 0, 1, 0, S, T, MAXLINES>(lds, nlines, lstride, tw);
+    fft_stages_ct<N, 0, 1, 0, S, T, MAXLINES, fft_shape_of(N).nstages>(lds, nlines, lstride, tw);
   } else {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     for (int line = wave; line < nlines; line += FFT_THREADS / 64) {

@@ -247,12 +247,13 @@ __host__ __device__ constexpr int assign_queue(int threads) { return threads * (
 //
 // The other half of the kernel is the lines: zeroing, conversion, FFT and
 // store.  A thread converts and stores cells of one line, with no index
-// division, all of them between two barriers.  Measured, float, before and
-// after both changes: N = 360 with 2e4 points 0.41 -> 0.30 ms, 1e6 0.563 ->
-// 0.478, 4e6 1.19 -> 1.09; N = 512, 4e6 2.16 -> 1.96; N = 256, 3e5 0.174 ->
-// 0.151; double, N = 360, 1e6 0.655 -> 0.553.  (Fixed point by adding 1.5 * 2^52
-// instead of the float64 conversion, under a branch on the weight's size: 0.51
-// -> 0.57 at N = 360.)
+// division, all of them between two barriers; at compile-time N the FFT's last
+// stage stores straight to the grid.  Measured, float, before and
+// after: N = 360 with 2e4 points 0.41 -> 0.30 ms, 1e6 0.563 -> 0.463 (0.475
+// without the last stage's stores), 4e6 1.19 -> 1.09; N = 512, 4e6 2.16 -> 1.88;
+// N = 256, 3e5 0.174 -> 0.151; double, N = 360, 1e6 0.655 -> 0.54.  (Fixed
+// point by adding 1.5 * 2^52 instead of the float64 conversion, under a branch on
+// the weight's size: 0.51 -> 0.57 at N = 360.)
 template <typename T, int NC, bool FFTX, int TH>
 __global__ __launch_bounds__(TH) void k_assign_lines(
     const float4* __restrict__ rec, const unsigned* __restrict__ tile_off, const AssignBoxes bs,
@@ -464,9 +465,17 @@ __global__ __launch_bounds__(TH) void k_assign_lines(
     cplx<T>* twl = lds + nl * lstride;
     stage_twiddles(twl, tw, N);
     __syncthreads();
-    fft_tile<NC, 1, T, assign_lines_max<T, NC>(), TileCfg<T>::ELEMS>(lds, sh, nl, lstride, twl);
-    if (stored)
-      for (int x = xf; x < N; x += TP) dst[x] = lds[line * lstride + x];
+    if constexpr (NC > 0) {
+      fft_tile_store<NC, 1, T, assign_lines_max<T, NC>()>(
+          lds, nl, lstride, twl, [&](int l, int n, cplx<T> v) {
+            const int y = y0 + l % at.ty, zz = z0 + l / at.ty;
+            if (y < y1 && zz < z1) out[((int64_t)zz * N + y) * N + n] = v;
+          });
+    } else {
+      fft_tile<NC, 1, T, assign_lines_max<T, NC>(), TileCfg<T>::ELEMS>(lds, sh, nl, lstride, twl);
+      if (stored)
+        for (int x = xf; x < N; x += TP) dst[x] = lds[line * lstride + x];
+    }
   }
 }
 
