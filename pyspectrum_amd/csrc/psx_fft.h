@@ -306,8 +306,9 @@ __device__ __forceinline__ void fft_stages_ct(cplx<T>* lds, int nlines, int lstr
 
 // The lines of the tile transformed, the last stage's butterflies not back to
 // LDS but to store(line, n, value): n = j + r N/R, so that a line's lanes hold
-// consecutive n (compile-time N).
-template <int N, int S, typename T, int MAXLINES, typename Store>
+// consecutive n (compile-time N), or, with COLUMNS, neighbouring lanes the same
+// n of neighbouring lines.
+template <int N, int S, typename T, int MAXLINES, bool COLUMNS, typename Store>
 __device__ __forceinline__ void fft_tile_store(cplx<T>* lds, int nlines, int lstride,
                                                const cplx<T>* __restrict__ tw, Store store) {
   constexpr FftShape sh = fft_shape_of(N);
@@ -317,7 +318,8 @@ __device__ __forceinline__ void fft_tile_store(cplx<T>* lds, int nlines, int lst
   fft_stages_ct<N, 0, 1, 0, S, T, MAXLINES, LAST>(lds, nlines, lstride, tw);
   // the earlier stages have NB - 1 twiddles (the sum of Ns (R - 1) telescopes)
   const cplx<T>* tl = tw + NB - 1;
-  const int line = (int)threadIdx.x / TPL, lane = (int)threadIdx.x - line * TPL;
+  const int line = COLUMNS ? (int)threadIdx.x % MAXLINES : (int)threadIdx.x / TPL;
+  const int lane = COLUMNS ? (int)threadIdx.x / MAXLINES : (int)threadIdx.x - line * TPL;
   const bool act = line < nlines;
   const cplx<T>* base = lds + line * lstride;
   cplx<T> v[MAXQ][R];

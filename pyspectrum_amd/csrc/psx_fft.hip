@@ -231,14 +231,27 @@ __global__ __launch_bounds__(FFT_THREADS) void k_shell_z(const cplx<T>* __restri
   cplx<T>* twl = lds + NL * lstride;
   stage_twiddles(twl, tw, N);
   __syncthreads();
-  fft_tile<NC, -1, T, NL, NL * 1024>(lds, sh, NL, lstride, twl);
-  cplx<T>* dst = T1 + sd.off[s] + (int64_t)ky * kxw + kx0 + c;
+  cplx<T>* dst = T1 + sd.off[s] + (int64_t)ky * kxw + kx0;
   const int64_t dstride = (int64_t)N * kxw;
-  for (int n = n0; n < N; n += RS) dst[(int64_t)n * dstride] = lds[c * lstride + n];
+  if constexpr (NC > 0) {
+    fft_tile_store<NC, -1, T, NL, true>(lds, NL, lstride, twl, [&](int line, int n, cplx<T> v) {
+      dst[n * dstride + line] = v;
+    });
+  } else {
+    fft_tile<NC, -1, T, NL, NL * 1024>(lds, sh, NL, lstride, twl);
+    for (int n = n0; n < N; n += RS) dst[n * dstride + c] = lds[c * lstride + n];
+  }
 }
 
 // y pass: tile (s, z, kx0): NL kx columns at one z; rows (ky, kx-tile) that
-// the z pass skipped (|ky| > kyl, the tile's c) are zero and not read.
+// the z pass skipped (|ky| > kyl, the tile's c) are zero and not read.  Both
+// passes move 8 to 16 bytes per value and direction and take most of their time for
+// that; the last FFT stage stores to memory with neighbouring lanes in
+// neighbouring columns (128-byte runs), without the LDS round trip.  Measured,
+// float: N = 360, 38 shells z 0.352 -> 0.331 ms, y 0.950 -> 0.925; N = 512, 60
+// shells z 0.893 -> 0.828, y 3.53 -> 3.31; double layers of N = 360 z 0.94 ->
+// 0.92, y 1.75 both.  (k_fft_lines the same way: N = 512 0.538 -> 0.516, but N =
+// 360 0.184 -> 0.187: left.)
 template <typename T, int NC>
 __global__ __launch_bounds__(FFT_THREADS) void k_shell_y(const cplx<T>* __restrict__ T1,
                                                          cplx<T>* __restrict__ T2,
@@ -279,9 +292,15 @@ __global__ __launch_bounds__(FFT_THREADS) void k_shell_y(const cplx<T>* __restri
   cplx<T>* twl = lds + NL * lstride;
   stage_twiddles(twl, tw, N);
   __syncthreads();
-  fft_tile<NC, -1, T, NL, NL * 1024>(lds, sh, NL, lstride, twl);
-  cplx<T>* dst = T2 + base + c;
-  for (int n = n0; n < N; n += RS) dst[(int64_t)n * kxw] = lds[c * lstride + n];
+  cplx<T>* dst = T2 + base;
+  if constexpr (NC > 0) {
+    fft_tile_store<NC, -1, T, NL, true>(lds, NL, lstride, twl, [&](int line, int n, cplx<T> v) {
+      dst[n * kxw + line] = v;
+    });
+  } else {
+    fft_tile<NC, -1, T, NL, NL * 1024>(lds, sh, NL, lstride, twl);
+    for (int n = n0; n < N; n += RS) dst[(int64_t)n * kxw + c] = lds[c * lstride + n];
+  }
 }
 
 // x pass (Hermitian -> real): tile (s, z, y0) covers rows y0..y0+2NP-1 as NP
@@ -353,7 +372,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_shell_x(const cplx<T>* __restri
   __syncthreads();
   if constexpr (NC > 0) {
     T* row = D + ((int64_t)s * N * N + (int64_t)z * N + y0) * N;
-    fft_tile_store<NC, -1, T, NP>(lds, npair, lstride, twl, [&](int line, int n, cplx<T> v) {
+    fft_tile_store<NC, -1, T, NP, false>(lds, npair, lstride, twl, [&](int line, int n, cplx<T> v) {
       row[2 * line * N + n] = v.re;
       row[(2 * line + 1) * N + n] = v.im;
     });

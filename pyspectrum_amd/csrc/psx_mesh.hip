@@ -466,7 +466,7 @@ __global__ __launch_bounds__(TH) void k_assign_lines(
     stage_twiddles(twl, tw, N);
     __syncthreads();
     if constexpr (NC > 0) {
-      fft_tile_store<NC, 1, T, assign_lines_max<T, NC>()>(
+      fft_tile_store<NC, 1, T, assign_lines_max<T, NC>(), false>(
           lds, nl, lstride, twl, [&](int l, int n, cplx<T> v) {
             const int y = y0 + l % at.ty, zz = z0 + l / at.ty;
             if (y < y1 && zz < z1) out[((int64_t)zz * N + y) * N + n] = v;
