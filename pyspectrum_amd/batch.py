@@ -34,7 +34,8 @@ def run_batch(ctx, xyzs, ws, Lboxes, Ngrid, step, Ncut, Nmax, precision, device,
     keep = []
     sums = []
     xs = [P._positions(x, device) for x in xyzs]
-    wds = P._weights_list([None] * nbox if ws is None else ws, [x.shape[1] for x in xs], device)
+    ws = [None if ws is None else ws[b] for b in range(nbox)]  # a short ws is an IndexError here
+    wds = P._weights_list(ws, [x.shape[1] for x in xs], device)
     for b, (x, (wd, sw, sabs)) in enumerate(zip(xs, wds)):
         n = x.shape[1]
         keep += [x, wd]
