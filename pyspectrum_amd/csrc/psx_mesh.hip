@@ -512,7 +512,19 @@ static int assign_lines_th(psx_ctx* ctx, const float4* rec, const unsigned* off,
 // N = 64, 2e4 0.018 -> 0.017, 2e6 0.60 -> 0.415; above, the wide ones lose what
 // is sparse: N = 80 (800 tiles) 2e4 0.026 -> 0.046, 5e5 0.168 -> 0.189, N = 128
 // 2e4 0.034 -> 0.056.
-constexpr int ASSIGN_WIDE_TILES = 512, ASSIGN_WIDE_THREADS = 1024;
+//
+// The double kernel of a run-time length needs all 128 registers of a thread
+// in a workgroup of 1024 and spills (40 bytes a lane), so a CU holds one: past
+// 256 tiles a second round starts, which costs more than the wide workgroups
+// gain until there is a particle a cell.  Measured, double, the whole field, 256
+// against 1024 threads at 0.02, 0.5, 0.9, 1, 2 and 8 particles a cell: N = 50
+// (325 tiles) 0.048 / 0.061, 0.106 / 0.111, 0.152 / 0.153, 0.164 / 0.163, 0.281 /
+// 0.268, 0.961 / 0.871 ms; N = 60 (450) 0.049 / 0.062, 0.122 / 0.126, 0.181 /
+// 0.183, 0.197 / 0.193, 0.339 / 0.325, 1.21 / 1.12.
+// Up to 256 tiles, N = 40 (200), at 0.02, 0.5 and 8: 0.042 -> 0.043, 0.079 ->
+// 0.069, 0.64 -> 0.49; compile-time N = 64 (512, no spill): 0.038 -> 0.040,
+// 0.116 -> 0.106, 1.29 -> 1.11.
+constexpr int ASSIGN_WIDE_TILES = 512, ASSIGN_WIDE_THREADS = 1024, ASSIGN_CUS = 256;
 
 template <typename T, int NC>
 static int assign_lines_n(psx_ctx* ctx, const float4* rec, const unsigned* off,
@@ -521,7 +533,11 @@ static int assign_lines_n(psx_ctx* ctx, const float4* rec, const unsigned* off,
   if (!fft_x)
     return assign_lines_th<T, 0, false, FFT_THREADS>(ctx, rec, off, bs, nbox, N, at, grid);
   if constexpr (NC <= 64) {
-    if ((int64_t)at.nty * at.ntz * nbox <= ASSIGN_WIDE_TILES)
+    const int64_t tiles = (int64_t)at.nty * at.ntz * nbox;
+    int64_t total = 0;
+    for (int b = 0; b < nbox; ++b) total += bs.np[b];
+    const bool second_round = sizeof(T) == 8 && NC == 0 && tiles > ASSIGN_CUS;
+    if (tiles <= ASSIGN_WIDE_TILES && (!second_round || total >= (int64_t)nbox * N * N * N))
       return assign_lines_th<T, NC, true, ASSIGN_WIDE_THREADS>(ctx, rec, off, bs, nbox, N, at, grid);
   }
   return assign_lines_th<T, NC, true, FFT_THREADS>(ctx, rec, off, bs, nbox, N, at, grid);
