@@ -106,6 +106,8 @@ def _weights_list(ws, ns, device):
         if w is None:
             out.append((None, float(n), float(n)))
         elif isinstance(w, torch.Tensor):
+            if w.numel() < n:  # the assignment reads n of them
+                raise ValueError("w must have shape (N,)")
             out.append((w.to(device=_device(device), dtype=torch.float32).contiguous(),))
             sums = _tensor_sums(w)
             if w.device == _device(device):
