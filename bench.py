@@ -168,12 +168,17 @@ def kernel_traffic(kernel, N, Nmax, prec):
 
 def roofline(box, prec, kern):
     """Roofline of the kernel with the most device time per box.  The
-    triangle sums are G * (Npairs + 2 Ntri) flops per launch (one product per
-    shell pair and point, one multiply-add per triangle and point); the fused
-    kernel also runs the x pass of the shell fields, 5 N log2(N) flops per
-    complex line of N points, ceil(Nshell / 2) lines per (y, z) row."""
+    triangle sums are G * (Npairs + 2 Ntri) flops per box (one product per
+    shell pair and point, one multiply-add per triangle and point) on G = N^3
+    points, in FP64 added up over the point sets that the kernel sums on
+    (psx_bk_layers); the fused kernel also runs the x pass of the shell fields,
+    5 N log2(N) flops per complex line of N points, ceil(Nshell / 2) lines per
+    (y, z) row."""
     name = max(kern, key=lambda k: kern[k]["ms_per_box"])
     N = box.N
+    k = kern[name]
+    traffic = kernel_traffic(name, N, box.Nmax, prec)
+    traffic_box = None if traffic is None else traffic * k["launches_per_box"]
     G = float(N) ** 3
     npairs = len({(int(i), int(j)) for i, j, _ in box.ijl})
     flops = G * (npairs + 2 * box.ntri)
@@ -182,15 +187,21 @@ def roofline(box, prec, kern):
         flops += 5.0 * G * np.log2(N) * ((ns + 1) // 2)
     elif name != "k_contract":
         return {"bound": None, "kernel": name, "achieved": None, "peak": None, "unit": None,
-                "frac": None, "traffic": kernel_traffic(name, N, box.Nmax, prec)}
-    t = kern[name]["ms_per_launch"] / 1e3
-    achieved = flops / t / 1e12
+                "frac": None, "traffic": traffic, "traffic_per_box": traffic_box}
+    elif prec == "fp64":
+        rows = box.L.layers(N, box.step, box.Ncut, box.Nmax)
+        if len(rows):
+            flops = sum(float(M) ** 3 * (float(np_) + 2.0 * nt) for M, _, nt, np_, mfma in rows if mfma)
+    achieved = flops / (k["ms_per_box"] / 1e3) / 1e12
     peak = PEAK["bf16_tflops"] if prec == "bf16x3" else (
         PEAK["fp32_tflops"] if prec == "fp32" else PEAK["fp64_tflops"])
+    assert achieved <= peak, "%s: %.1f TFLOP/s counted, the peak is %.1f" % (name, achieved, peak)
     return {"bound": "mfma", "kernel": name, "achieved": round(achieved, 2), "peak": peak,
             "unit": "TFLOP/s", "frac": round(achieved / peak, 4),
-            "flops_per_launch": flops, "ms_per_launch": round(kern[name]["ms_per_launch"], 4),
-            "traffic": kernel_traffic(name, N, box.Nmax, prec)}
+            "flops_per_launch": flops / k["launches_per_box"],
+            "ms_per_launch": round(k["ms_per_launch"], 4), "traffic": traffic,
+            "flops_per_box": flops, "ms_per_box": round(k["ms_per_box"], 4),
+            "traffic_per_box": traffic_box}
 
 
 def host_cores():

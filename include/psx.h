@@ -232,6 +232,14 @@ int psx_apply_rsd(psx_ctx* ctx, const float* xyz, const float* v, int64_t np, do
 int psx_bk_num_triangles(int step, int ncut, int nmax, int64_t* ntri /* [host] */);
 int psx_bk_triangles(int step, int ncut, int nmax, int32_t* ijl /* [host] [ntri][3] */);
 
+/* The point sets of the FP64 triangle sums of a shape, up to three rows (M,
+ * 1 if shifted by half a cell, triangles, their distinct (i, j) pairs, 1 if
+ * summed on the matrix cores) of M^3 points each; *n = 0: all triangles on the
+ * ngrid^3 grid.  (No reference counterpart: it sums every triangle on the
+ * grid.) */
+int psx_bk_layers(int ngrid, int step, int ncut, int nmax, int32_t* rows /* [host] [3][5] */,
+                  int* n /* [host] */);
+
 /* Replaces the shell loop of _Bk_periodic (pyspectrum.py:387-400):
  * d_j(x) = Re FFT_forward[delta * 1(shell == j)] for j = Ncut//step..Nmax,
  * written as real [ns][N^3] (float for F32/BF16X3, double for F64). */

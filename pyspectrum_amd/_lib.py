@@ -64,6 +64,7 @@ SIGNATURES = {
     "psx_apply_rsd": [_p, _p, _p, _i64, _d, _d, _i, _p],
     "psx_bk_num_triangles": [_i, _i, _i, _c.POINTER(_i64)],
     "psx_bk_triangles": [_i, _i, _i, _p],
+    "psx_bk_layers": [_i, _i, _i, _i, _p, _c.POINTER(_i)],
     "psx_bk_shell_fields": [_p, _p, _i, _i, _i, _i, _p, _i],
     "psx_bk_contract": [_p, _p, _i, _i, _i, _i, _p, _i],
     "psx_bk_raw": [_p, _p, _i, _i, _i, _i, _p, _p, _i],
@@ -243,4 +244,13 @@ def triangles(step, Ncut, Nmax):
     call("psx_bk_num_triangles", step, Ncut, Nmax, ctypes.byref(n))
     out = np.zeros((max(n.value, 1), 3), dtype=np.int32)
     call("psx_bk_triangles", step, Ncut, Nmax, out.ctypes.data_as(_p))
+    return out[: n.value]
+
+
+def layers(Ngrid, step, Ncut, Nmax):
+    """Point sets of the FP64 triangle sums (host): int32 rows (M, shifted,
+    triangles, (i, j) pairs, on the matrix cores); none: all on the Ngrid^3 grid."""
+    n = _i()
+    out = np.zeros((3, 5), dtype=np.int32)
+    call("psx_bk_layers", Ngrid, step, Ncut, Nmax, out.ctypes.data_as(_p), ctypes.byref(n))
     return out[: n.value]

@@ -4,6 +4,7 @@
 #include <cstring>
 #include <mutex>
 #include <numeric>
+#include <set>
 
 #include "psx_ctx.h"
 #include "psx_lattice.h"
@@ -296,12 +297,8 @@ int get_contract_plan(psx_ctx* ctx, int prec, int step, int ncut, int nmax,
 }
 
 // ---------------------------------------------------------- FP64 layers ----
-int get_lattice_plan(psx_ctx* ctx, int N, int step, int ncut, int nmax, const LatticePlan** out) {
-  auto key = std::make_tuple(N, step, ncut, nmax);
-  auto it = ctx->lattice_plans.find(key);
-  if (it != ctx->lattice_plans.end()) { *out = it->second.get(); return PSX_OK; }
-  std::vector<int> ijl, sizes;
-  triangle_list(step, ncut, nmax, &ijl);
+static std::vector<LayerChoice> lattice_choice(const std::vector<int>& ijl, int N, int step) {
+  std::vector<int> sizes;
 #define PSX_ADD_N(n) sizes.push_back(n);
   PSX_LAT_SIZES(PSX_ADD_N)
 #undef PSX_ADD_N
@@ -310,9 +307,23 @@ int get_lattice_plan(psx_ctx* ctx, int N, int step, int ncut, int nmax, const La
 #define PSX_IF_N(n) fast = fast || N == n;
   PSX_FFT_SIZES(PSX_IF_N)
 #undef PSX_IF_N
+  return choose_layers(ijl, N, [&](int j) { return shell_mmax(j, step); }, sizes, fast);
+}
+
+// Whether a layer's few triangles on few shells are summed without the
+// matrix cores (k_tri_direct).
+static bool direct_layer(int ntri, int nshells) {
+  return ntri <= DIRECT_TRI && nshells <= DIRECT_SHELLS;
+}
+
+int get_lattice_plan(psx_ctx* ctx, int N, int step, int ncut, int nmax, const LatticePlan** out) {
+  auto key = std::make_tuple(N, step, ncut, nmax);
+  auto it = ctx->lattice_plans.find(key);
+  if (it != ctx->lattice_plans.end()) { *out = it->second.get(); return PSX_OK; }
+  std::vector<int> ijl;
+  triangle_list(step, ncut, nmax, &ijl);
   auto lp = std::make_unique<LatticePlan>();
-  for (const LayerChoice& c :
-       choose_layers(ijl, N, [&](int j) { return shell_mmax(j, step); }, sizes, fast)) {
+  for (const LayerChoice& c : lattice_choice(ijl, N, step)) {
     LatticeLayer l;
     l.M = c.M;
     l.add = c.add;
@@ -335,7 +346,7 @@ int get_lattice_plan(psx_ctx* ctx, int N, int step, int ncut, int nmax, const La
     }
     PSX_TRY(upload(ctx, c.tri, &l.d_map));
     PSX_TRY(upload(ctx, c.weight, &l.d_weight));
-    if (l.ntri > DIRECT_TRI || l.nmax - l.j0 + 1 > DIRECT_SHELLS) {
+    if (!direct_layer(l.ntri, l.nmax - l.j0 + 1)) {
       l.cp = std::make_unique<ContractPlan>();
       PSX_TRY(build_contract_plan(ctx, PSX_PREC_F64, false, l.ijl, l.j0, l.nmax, l.cp.get()));
     }
@@ -820,6 +831,29 @@ int psx_bk_triangles(int step, int ncut, int nmax, int32_t* out) {
   std::vector<int> ijl;
   triangle_list(step, ncut, nmax, &ijl);
   std::memcpy(out, ijl.data(), ijl.size() * sizeof(int32_t));
+  return PSX_OK;
+}
+
+int psx_bk_layers(int ngrid, int step, int ncut, int nmax, int32_t* rows, int* n) {
+  PSX_REQUIRE(rows && n, "null argument");
+  PSX_TRY(check_bk_args(ngrid, step, ncut, nmax));
+  std::vector<int> ijl;
+  triangle_list(step, ncut, nmax, &ijl);
+  *n = 0;
+  for (const LayerChoice& c : lattice_choice(ijl, ngrid, step)) {
+    std::set<std::pair<int, int>> pairs;
+    int lo = nmax, hi = 0;
+    for (int t : c.tri) {
+      pairs.insert({ijl[3 * t], ijl[3 * t + 1]});
+      lo = std::min(lo, ijl[3 * t + 2]);
+      hi = std::max(hi, ijl[3 * t]);
+    }
+    const int ntri = (int)c.tri.size();
+    const int32_t r[5] = {c.M, c.shifted ? 1 : 0, ntri, (int32_t)pairs.size(),
+                          direct_layer(ntri, hi - lo + 1) ? 0 : 1};
+    std::memcpy(rows + 5 * *n, r, sizeof r);
+    ++*n;
+  }
   return PSX_OK;
 }
 
