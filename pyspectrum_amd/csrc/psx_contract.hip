@@ -655,9 +655,11 @@ int launch_contract(psx_ctx* ctx, const void* D, int N, int step, int ncut, int 
 
 // ----------------------------------------------------------- finalize -----
 // _Bk_periodic (pyspectrum.py:418-445) and Bk_periodic (:346-355) in float64.
-// tri: [ntri][3] shell indices (i, j, l); p0k[j-1]; cnt[t] = the normalisation
-// sum_x I_i I_j I_l.  Zero-count triangles produce zeros before the unit
-// conversion, as in the reference.
+// tri: [ntri][3] shell indices (i, j, l); p0k[j-1], for shell 0 (Ncut < step)
+// the last entry, as the reference's index -1 reads it (the list ends with the
+// triangle of the last shell); cnt[t] = the normalisation sum_x I_i I_j I_l.
+// Zero-count triangles produce zeros before the unit conversion, as in the
+// reference.
 // Box blockIdx.y of a batch: braw [box][ntri], p0k [box][p0k_stride],
 // out [box][7][ntri], its own nbar and kf^3, kf^6.
 struct BkConst {
@@ -684,7 +686,9 @@ __global__ void k_bk_finalize(const double* __restrict__ braw, const double* __r
   const double n = cnt[t];
   double p1 = 0, p2 = 0, p3 = 0, b = 0, cc = 0;
   if (n > 0) {
-    p1 = p0k[i - 1]; p2 = p0k[j - 1]; p3 = p0k[l - 1];
+    const int nmax = tri[3 * (ntri - 1)];
+    auto power = [&](int s) { return p0k[(s > 0 ? s : nmax) - 1]; };
+    p1 = power(i); p2 = power(j); p3 = power(l);
     b = braw[t] / n;
     cc = n / (fac * c.G);
   }
