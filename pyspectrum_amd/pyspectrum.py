@@ -154,6 +154,14 @@ def _check_ngrid(Ngrid):
         raise ValueError("Ngrid must be even")
 
 
+def _full_field(delta):
+    """A full field as a tensor; the device reads it by its strides as a cube."""
+    d = delta if isinstance(delta, torch.Tensor) else torch.from_numpy(np.asarray(delta))
+    if d.dim() != 3 or len(set(d.shape)) != 1:
+        raise ValueError("delta must have shape (Ngrid, Ngrid, Ngrid)")
+    return d
+
+
 # ------------------------------------------------------------- front end ----
 def FFT_periodic(xyz, w=None, Lbox=2600., Ngrid=360, fft='pyfftw', silent=True, precision='fp32',
                  device=0):
@@ -433,7 +441,7 @@ def _Bk_periodic(delta, Nmax=40, Ncut=3, step=3, fft='pyfftw', nthreads=1, silen
     """Bispectrum of a full delta(k) field, before units and shot noise
     (pyspectrum.py:359-457).  ``delta``: (Ngrid, Ngrid, Ngrid) complex [ix, iy, iz].
     """
-    d = delta if isinstance(delta, torch.Tensor) else torch.from_numpy(np.asarray(delta))
+    d = _full_field(delta)
     Ngrid = d.shape[0]
     _check_ngrid(Ngrid)
     prec = _prec(precision)
@@ -590,7 +598,7 @@ def _B0_survey(delta, alpha, I12, I13, I22, I23, I33, Nmax=40, Ncut=3, step=3, f
     """Survey bispectrum monopole of a full delta(k) = delta_data - alpha
     delta_random (pyspectrum.py:135-282).  ``delta``: (Ngrid, Ngrid, Ngrid)
     complex [ix, iy, iz]; the I's are the random catalogue's sums times alpha."""
-    d = delta if isinstance(delta, torch.Tensor) else torch.from_numpy(np.asarray(delta))
+    d = _full_field(delta)
     Ngrid = d.shape[0]
     _check_ngrid(Ngrid)
     prec = _prec(precision)
