@@ -117,7 +117,6 @@ struct ContractPlan {
   int* d_pair_s = nullptr;              // [npt*16][2] shell slots (i-j0, j-j0) per row (-1 pad)
   int* d_tri_loc = nullptr;             // [ntri] slot*256 + lane*4 + reg
   int* d_tri_grp = nullptr;             // [ntri] group of the triangle's pair tile
-  int* d_tri_ijl = nullptr;             // [ntri][3] shell indices i, j, l (reference loop order)
 };
 
 // One point set of the FP64 triangle sums (psx_lattice.h) with the triangles

@@ -355,7 +355,7 @@ __device__ __forceinline__ void fft_tile_store(cplx<T>* lds, int nlines, int lst
 // Runtime N: one wave per line, 64 butterflies a pass, so a line's stages need
 // no workgroup barrier (a wave's LDS accesses are carried out in order) and the
 // register arrays stay small for any N <= FFT_MAX_N.  (The threads of a
-// workgroup sharing all lines, as below for compile-time N, needs arrays sized
+// workgroup sharing all lines, as above for compile-time N, needs arrays sized
 // for the worst N, 190 to 256 registers.  Measured at N = 300, float: y pass
 // 0.37 -> 0.15 ms, assignment 0.66 -> 0.38, shell y pass of 20 shells 0.50 ->
 // 0.28, shell x pass 3.9 -> 1.02.  At compile-time N the shared form stays: with
@@ -415,7 +415,7 @@ __device__ __forceinline__ void fft_stage_wave(cplx<T>* base, int N, int Ns,
 
 // Transform every line of the tile in place.  N > 0: compile-time length;
 // N == 0: runtime length sh.N.
-template <int N, int S, typename T, int MAXLINES, int TILE_ELEMS>
+template <int N, int S, typename T, int MAXLINES>
 __device__ __forceinline__ void fft_tile(cplx<T>* lds, const FftShape& sh, int nlines, int lstride,
                                          const cplx<T>* __restrict__ tw) {
   if constexpr (N > 0) {
@@ -462,7 +462,8 @@ inline void fft_stage_twiddles(const FftShape& sh, const C* full /* exp(-2 pi i 
 // Sizes with a compile-time instantiation; others run the runtime-N engine.
 #define PSX_FFT_SIZES(X) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(360) X(384) X(512)
 // Grid lengths of the FP64 point sets (psx_lattice.h): those and a few
-// between, so that the smallest that fits is at most a quarter too long.
+// between.  Neighbours are a quarter apart or less, except 32 to 48 (a half) and
+// 48 to 64, 96 to 128 and 384 to 512 (a third).
 #define PSX_LAT_SIZES(X) PSX_FFT_SIZES(X) X(80) X(160) X(240) X(288) X(320)
 
 }  // namespace psx

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_fft_lines(
   cplx<T>* twl = lds + tl * lstride;
   stage_twiddles(twl, tw, N);
   __syncthreads();
-  fft_tile<NC, S, T, Tile<T, NC>::MAXLINES, TileCfg<T>::ELEMS>(lds, sh, nl, lstride, twl);
+  fft_tile<NC, S, T, Tile<T, NC>::MAXLINES>(lds, sh, nl, lstride, twl);
   for (int idx = threadIdx.x; idx < tl * N; idx += FFT_THREADS) {
     int c, n;
     if (es == 1) { c = idx / N; n = idx - c * N; }
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_shell_z(const cplx<T>* __restri
       dst[n * dstride + line] = v;
     });
   } else {
-    fft_tile<NC, -1, T, NL, NL * 1024>(lds, sh, NL, lstride, twl);
+    fft_tile<NC, -1, T, NL>(lds, sh, NL, lstride, twl);
     for (int n = n0; n < N; n += RS) dst[n * dstride + c] = lds[c * lstride + n];
   }
 }
@@ -298,7 +298,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_shell_y(const cplx<T>* __restri
       dst[n * kxw + line] = v;
     });
   } else {
-    fft_tile<NC, -1, T, NL, NL * 1024>(lds, sh, NL, lstride, twl);
+    fft_tile<NC, -1, T, NL>(lds, sh, NL, lstride, twl);
     for (int n = n0; n < N; n += RS) dst[(int64_t)n * kxw + c] = lds[c * lstride + n];
   }
 }
@@ -377,7 +377,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_shell_x(const cplx<T>* __restri
       row[(2 * line + 1) * N + n] = v.im;
     });
   } else {
-    fft_tile<NC, -1, T, NP, NP * 1024>(lds, sh, npair, lstride, twl);
+    fft_tile<NC, -1, T, NP>(lds, sh, npair, lstride, twl);
     // rows y0 .. y0 + 2 npair - 1 are contiguous in D: one coalesced stream
     const int64_t G = (int64_t)N * N * N;
     T* dst = D + (int64_t)s * G + ((int64_t)z * N + y0) * N;

@@ -42,6 +42,13 @@ struct LayerChoice {
 // for 40 shells; lengths without a compile-time FFT take about twice the
 // latter), plus its launches.  At most DIRECT_TRI triangles on DIRECT_SHELLS
 // shells are summed directly, in one read of the fields.
+// Measured against the N^3 grid (psx_bk_raw and the shell fields with their
+// contraction, N = 48 to 512): every one of 18 shapes that take layers is faster,
+// by 1.3 (256 / step 2 / 44 shells, 8.35 against 10.9 ms) to 4.9 (512 / 2 / 60).
+// The rule errs towards the grid: with layers forced, 14 of 28 shapes that it
+// leaves there were slower (96 / 3 / 12 0.81, 256 / 3 / 30 0.81, 200 / 3 / 24 0.79),
+// but 216 / 3 / 24, 192 / 6 / 9, 128 / 3 / 12 and 240 / 2 / 40 were 1.4 to 1.5 times
+// as fast.
 constexpr int DIRECT_TRI = 16, DIRECT_SHELLS = 8;
 inline double layer_cost(double G, int ntri, int nshells, bool fast_fft) {
   const double blocks = std::max(4.0, 1.65 * ntri / 256.0 + 4.0);

@@ -410,7 +410,10 @@ __global__ __launch_bounds__(TH) void k_assign_lines(
     __syncthreads();
   }
   __syncthreads();
-  if (TH > FFT_THREADS && threadIdx.x >= FFT_THREADS) return;  // whole waves: barriers go on without them
+  // The waves past the lines' threads end here, whole waves as TH and FFT_THREADS
+  // are multiples of 64, and the barriers below are the others': S_BARRIER waits
+  // for the waves of the workgroup that have not ended (CDNA3 and CDNA4 ISA).
+  if (TH > FFT_THREADS && threadIdx.x >= FFT_THREADS) return;
   // a thread converts and stores the cells x = x0, x0 + TP, ... of one line
   const double inv = 1.0 / scale;
   const int TP = FFT_THREADS / nl;
@@ -472,7 +475,7 @@ __global__ __launch_bounds__(TH) void k_assign_lines(
             if (y < y1 && zz < z1) out[((int64_t)zz * N + y) * N + n] = v;
           });
     } else {
-      fft_tile<NC, 1, T, assign_lines_max<T, NC>(), TileCfg<T>::ELEMS>(lds, sh, nl, lstride, twl);
+      fft_tile<NC, 1, T, assign_lines_max<T, NC>()>(lds, sh, nl, lstride, twl);
       if (stored)
         for (int x = xf; x < N; x += TP) dst[x] = lds[line * lstride + x];
     }
@@ -768,8 +771,8 @@ __global__ __launch_bounds__(256) void k_fcomb(const cplx<T>* __restrict__ F, cp
 // iteration (x, |y|, |z|) reads or leaves at (x, y, z) lies on one of them
 // (where x, y or z alias, the other lines of the iteration coincide with
 // these two).  A tile holds tp such line pairs, consecutive x at one y; the
-// line transforms are those of k_fft_lines, the combination that of k_fcomb.
-//
+// line transforms are those of k_fft_lines.  An element is formed from its two
+// values and fcomb_survivor instead of the eight stores that k_fcomb replays.
 //
 // The lines fill the LDS (two or three workgroups a CU), so between loads and
 // stores the kernel is bound by its own instructions and latencies.  A thread
@@ -828,7 +831,7 @@ __global__ __launch_bounds__(FFT_THREADS) void k_fft_zcomb(const cplx<T>* __rest
   cplx<T>* twl = lds + tl * lstride;
   stage_twiddles(twl, tw, N);
   __syncthreads();
-  fft_tile<NC, 1, T, ML, TileCfg<T>::ELEMS>(lds, sh, 2 * np, lstride, twl);
+  fft_tile<NC, 1, T, ML>(lds, sh, 2 * np, lstride, twl);
   // epilogue: pair c, rows z0, z0 + RZ, ...
   const int RZ = FFT_THREADS / tp;
   const int zfirst = (int)threadIdx.x / tp, c = (int)threadIdx.x - zfirst * tp;
